@@ -949,149 +949,418 @@ struct RowArgs {
   long offset;  // cached forward: T query rows at positions offset .. offset+T-1, keys 0 .. offset+T-1
 };
 
+// The row kernels (fp32, and bf16 shapes outside the MFMA layout): any even
+// head_dim up to 128, any window.  Their first form gave one wave a row and
+// walked its keys one at a time (a dot product over the lanes, a six-step
+// wave sum, the exponential, the accumulate): a serial chain of about 60 ns
+// a key, at most half the lanes in use below head_dim 64.  Here a workgroup
+// stages 64 streamed rows (keys, or queries for dK | dV) in LDS and each wave
+// takes R fixed rows against them in two phases.  First lane j forms streamed
+// row j's whole dot product, and the softmax terms of 64 rows at once; then
+// the lanes turn to the columns (64 / C rows of C columns at a time) and add
+// the weighted rows one after another.  Every sum keeps the first form's
+// order (the dot product's pairwise tree over the columns, keys in order, the
+// running maximum after each key as a prefix maximum), so the results have
+// its bits, and a row's bits depend on its position alone: the cached forward
+// equals the full one.  The bound is now vector issue (two or three operations
+// a key and column, no sum over lanes).  fp32 training steps, whole: one layer
+// of d 128 on 2 x 128 tokens 200 -> 128 us; three of d 256 on 4 x 300 tokens
+// 2549 -> 765 us; two of d 128 (head_dim 64) on 6 x 250 tokens 666 -> 318 us.
+constexpr int RT_KEYS = 64;
+
+// C: the columns staged, the least power of two >= head_dim (4 at least); the
+// LDS row stride is C + 4 floats, so that 16 lanes reading 16 rows' chunk c
+// hit distinct banks
+template <int C, int R>
+constexpr size_t rt_lds_bytes(int bwd) {
+  return sizeof(float) * ((size_t)(C + 4) * (2 * RT_KEYS + 4 * R * (1 + bwd)) + (size_t)8 * R * RT_KEYS);
+}
+
+// rows [row0, row0 + n) of a head's columns as fp32 into LDS; rows past
+// `last` repeat it (their terms are masked), columns past D are 0
+template <int C>
+__device__ __forceinline__ void rt_stage(float* dst, int n, const void* src, int dt, long sld, long row0, long last, long D,
+                                         bool vec) {
+  for (int i = threadIdx.x; i < n * (C / 4); i += 256) {
+    const int r = i / (C / 4), c = (i % (C / 4)) * 4;
+    const long row = row0 + r < last ? row0 + r : last;
+    float4 v;
+    if (vec && c + 4 <= D) {
+      if (dt == SJ_BF16) {
+        const u32x2 w = *(const u32x2*)((const bf16_t*)src + row * sld + c);
+        v = make_float4(__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u), __uint_as_float(w[1] << 16),
+                        __uint_as_float(w[1] & 0xffff0000u));
+      } else {
+        v = *(const float4*)((const float*)src + row * sld + c);
+      }
+    } else {
+      float e[4];
+      for (int k = 0; k < 4; k++) e[k] = c + k < D ? load_as_f32(src, dt, row * sld + c + k) : 0.f;
+      v = make_float4(e[0], e[1], e[2], e[3]);
+    }
+    *(float4*)(dst + r * (C + 4) + c) = v;
+  }
+}
+
+// 4-element vector loads of a head's columns (its base, the row stride and
+// the head width must keep them whole)
+__device__ __forceinline__ bool rt_vec(const void* p, int dt, long ld, long D) {
+  return D % 4 == 0 && ld % 4 == 0 && ((uintptr_t)p & (dt == SJ_BF16 ? 7 : 15)) == 0;
+}
+
+// The pairwise tree of a dot product: column d first meets d + L / 2 (L: the
+// lesser of C and 64), then d + L / 4, ...; column d + 64 joins column d's
+// product before the tree.  This call: the N chunks (4 columns) c0, c0 + S, ...
+template <int C, int N, int S, int R>
+__device__ __forceinline__ void rt_tree(const float* A, const float* x, int c0, float4* out) {
+  if constexpr (N == 1) {
+    const float4 v = *(const float4*)(x + 4 * c0);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const float4 q = *(const float4*)(A + r * (C + 4) + 4 * c0);
+      out[r] = make_float4(mul_rn(q.x, v.x), mul_rn(q.y, v.y), mul_rn(q.z, v.z), mul_rn(q.w, v.w));
+    }
+    if constexpr (C > 64) {
+      const float4 u = *(const float4*)(x + 4 * c0 + 64);
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const float4 q = *(const float4*)(A + r * (C + 4) + 4 * c0 + 64);
+        out[r] = make_float4(fmaf(q.x, u.x, out[r].x), fmaf(q.y, u.y, out[r].y), fmaf(q.z, u.z, out[r].z),
+                             fmaf(q.w, u.w, out[r].w));
+      }
+    }
+  } else {
+    float4 o[R];
+    rt_tree<C, N / 2, 2 * S, R>(A, x, c0, out);
+    rt_tree<C, N / 2, 2 * S, R>(A, x, c0 + S, o);
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      out[r] = make_float4(out[r].x + o[r].x, out[r].y + o[r].y, out[r].z + o[r].z, out[r].w + o[r].w);
+  }
+}
+template <int C, int R>
+__device__ __forceinline__ void rt_dots(const float* A, const float* x, float* s) {
+  float4 t[R];
+  rt_tree<C, (C > 64 ? 16 : C / 4), 1, R>(A, x, 0, t);
+#pragma unroll
+  for (int r = 0; r < R; r++) s[r] = (t[r].x + t[r].z) + (t[r].y + t[r].w);
+}
+
+// body(j, masked) over the streamed rows [j0, j1] of a tile that some fixed
+// row of the wave sees; all of them see [ja, jb]
+template <class F>
+__device__ __forceinline__ void rt_walk(long j0, long ja, long jb, long j1, F body) {
+  auto clip = [](long j) { return j < 0 ? 0 : j > RT_KEYS - 1 ? RT_KEYS - 1 : (int)j; };
+  const int b0 = clip(j0), b1 = clip(j1);
+  if (ja > jb || ja > RT_KEYS - 1 || jb < 0) {
+    for (int j = b0; j <= b1; j++) body(j, true);
+    return;
+  }
+  const int c0 = clip(ja), c1 = clip(jb);
+  for (int j = b0; j < c0; j++) body(j, true);
+#pragma unroll 8
+  for (int j = c0; j <= c1; j++) body(j, false);
+  for (int j = c1 + 1; j <= b1; j++) body(j, true);
+}
+
 // CACHED: the query rows of one sequence continue a KV cache (hierarchy.py:
 // 7-39 with OFFSET): row r sits at position offset + r and reads key rows
-// 0 .. offset + r; each row takes the same operations in the same order as
-// in the full forward, so the two agree bit for bit.
-template <bool CACHED>
+// 0 .. offset + r.  The lanes of column group g = lane / L (L the lesser of C
+// and 64) hold rows g, g + 64 / L, ... of the wave's R.
+template <int C, int R, bool CACHED>
 __global__ __launch_bounds__(256) void k_attn_fwd_rows(RowArgs a) {
-  const int lane = threadIdx.x & 63;
-  const long row = blockIdx.x * 4L + (threadIdx.x >> 6);  // (b*T + pos)*HQ + h
-  if (row >= a.B * a.T * a.HQ) return;
-  const long h = row % a.HQ, bt = row / a.HQ, pos = CACHED ? a.offset + bt : bt % a.T, b = CACHED ? 0 : bt / a.T;
-  const long kvh = h / (a.HQ / a.HK);
+  constexpr int L = C < 64 ? C : 64, G = 64 / L, RL = (R + G - 1) / G, LD = C + 4;
+  constexpr bool TWO = C > 64;  // a second column per lane
+  extern __shared__ __attribute__((aligned(16))) float rt[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float *X = rt, *Y = X + RT_KEYS * LD, *A = Y + RT_KEYS * LD, *P = A + 4 * R * LD;
+  // block of 4 R rows slowest, the last (longest walks) first
+  const long nblk = (a.T + 4 * R - 1) / (4 * R), per = a.HQ * a.B, id = blockIdx.x;
+  const long blk = nblk - 1 - id / per, h = (id % per) / a.B, b = id % a.B;
+  const long kvh = h / (a.HQ / a.HK), q0 = blk * 4 * R, off = CACHED ? a.offset : 0;
   const float scale = 1.f / sqrtf((float)a.D);
-  float q[2], acc[2] = {0.f, 0.f};
-  for (int i = 0; i < 2; i++) {
-    long d = lane + 64 * i;
-    q[i] = d < a.D ? load_as_f32(a.q, a.dt, bt * a.ldq + h * a.D + d) : 0.f;
-  }
-  float m = -INFINITY, l = 0.f;
-  long first = a.window > 0 ? (pos + 1 - a.window > 0 ? pos + 1 - a.window : 0) : 0;
-  for (long p = first; p <= pos; p++) {
-    long kr = (b * a.T + p);
-    float s = 0.f;
-    for (int i = 0; i < 2; i++) {
-      long d = lane + 64 * i;
-      if (d < a.D) s += q[i] * load_as_f32(a.k, a.dt, kr * a.ldk + kvh * a.D + d);
-    }
-    s = wave_sum(s) * scale;
-    float mn = fmaxf(m, s);
-    float al = expf(m - mn), pr = expf(s - mn);
-    for (int i = 0; i < 2; i++) {
-      long d = lane + 64 * i;
-      float vv = d < a.D ? load_as_f32(a.v, a.dt, kr * a.ldv + kvh * a.D + d) : 0.f;
-      acc[i] = acc[i] * al + pr * vv;
-    }
-    l = l * al + pr;
-    m = mn;
-  }
-  for (int i = 0; i < 2; i++) {
-    long d = lane + 64 * i;
-    if (d < a.D) store_from_f32(a.out, a.dt, bt * a.ldo + h * a.D + d, acc[i] / l);
-  }
-  if (!CACHED && lane == 0) a.lse[row] = m + logf(l);
-}
-
-__device__ __forceinline__ void inv_rope_store(float* dst, const float* rope, long pos, long D, int lane, float x0,
-                                               float x1) {
-  // lanes hold consecutive columns; pair partner is lane ^ 1 (D even)
-  float y0 = __shfl_xor(x0, 1, 64), y1 = __shfl_xor(x1, 1, 64);
-  float xs[2] = {x0, x1}, ys[2] = {y0, y1};
-  for (int i = 0; i < 2; i++) {
-    long d = lane + 64 * i;
-    if (d < D) {
-      float x = xs[i];
-      if (rope) {
-        float2 cs = *(const float2*)(rope + 2 * (pos * (D / 2) + (d >> 1)));
-        x = (d & 1) ? (x * cs.x - ys[i] * cs.y) : (x * cs.x + ys[i] * cs.y);
+  const size_t es = a.dt == SJ_BF16 ? 2 : 4;
+  const char* qh = (const char*)a.q + h * a.D * es;
+  const char *kh = (const char*)a.k + kvh * a.D * es, *vh = (const char*)a.v + kvh * a.D * es;
+  rt_stage<C>(A, 4 * R, qh, a.dt, a.ldq, b * a.T + q0, b * a.T + a.T - 1, a.D, rt_vec(qh, a.dt, a.ldq, a.D));
+  const bool kvec = rt_vec(kh, a.dt, a.ldk, a.D), vvec = rt_vec(vh, a.dt, a.ldv, a.D);
+  const long qlast = (q0 + 4 * R < a.T ? q0 + 4 * R : a.T) - 1;
+  const long kbase = CACHED ? 0 : b * a.T, klast = kbase + off + a.T - 1;
+  auto first = [&](long pos) { return a.window > 0 && pos + 1 > a.window ? pos + 1 - a.window : 0L; };
+  const int d = lane & (L - 1), g = lane / L;
+  const bool two = TWO && d + 64 < a.D;
+  float acc[RL][2], l[RL], m[R];
+#pragma unroll
+  for (int i = 0; i < RL; i++) acc[i][0] = acc[i][1] = l[i] = 0.f;
+#pragma unroll
+  for (int r = 0; r < R; r++) m[r] = -INFINITY;
+  const float* Aw = A + wave * R * LD;
+  float2* Pw = (float2*)P + wave * R * RT_KEYS;  // (probability, rescale) per row and key
+  const long w0 = q0 + wave * R;                 // the wave's first row
+  const long wl = w0 + R - 1 < qlast ? w0 + R - 1 : qlast;
+  for (long k0 = first(off + q0); k0 <= off + qlast; k0 += RT_KEYS) {
+    __syncthreads();
+    rt_stage<C>(X, RT_KEYS, kh, a.dt, a.ldk, kbase + k0, klast, a.D, kvec);
+    rt_stage<C>(Y, RT_KEYS, vh, a.dt, a.ldv, kbase + k0, klast, a.D, vvec);
+    __syncthreads();
+    if (w0 > qlast || k0 > off + wl || k0 + RT_KEYS <= first(off + w0)) continue;  // no visible key for this wave
+    float s[R];
+    rt_dots<C, R>(Aw, X + lane * LD, s);
+    const long p = k0 + lane;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const long pos = off + w0 + r;
+      const bool in = p >= first(pos) && p <= pos;
+      // the running maximum after this lane's key, and after the one before
+      float mx = in ? mul_rn(s[r], scale) : -INFINITY;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const float t = __shfl_up(mx, o, 64);
+        mx = lane >= o ? fmaxf(mx, t) : mx;
       }
-      dst[d] = x;
+      mx = fmaxf(m[r], mx);
+      const float t = __shfl_up(mx, 1, 64), before = lane ? t : m[r];
+      Pw[r * RT_KEYS + lane] = make_float2(expf(fmaf(scale, s[r], -mx)), expf(before - mx));
+      m[r] = __shfl(mx, 63, 64);
+    }
+    __builtin_amdgcn_wave_barrier();
+    // this lane's rows' visible keys of the tile
+    const float2* Pl[RL];
+    int lo[RL], hi[RL];
+#pragma unroll
+    for (int i = 0; i < RL; i++) {
+      const int r = g + i * G < R ? g + i * G : R - 1;
+      const long pos = off + w0 + r, f = first(pos);
+      Pl[i] = Pw + r * RT_KEYS;
+      lo[i] = f > k0 ? (int)(f - k0) : 0;
+      hi[i] = pos - k0 < RT_KEYS ? (int)(pos - k0) : RT_KEYS;
+    }
+    rt_walk(first(off + w0) - k0, first(off + wl) - k0, off + w0 - k0, off + wl - k0, [&](int j, bool masked) {
+      const float x0 = Y[j * LD + d], x1 = TWO ? Y[j * LD + d + 64] : 0.f;
+#pragma unroll
+      for (int i = 0; i < RL; i++) {
+        const float2 w = Pl[i][j];
+        const bool in = !masked || (j >= lo[i] && j <= hi[i]);
+        l[i] = in ? fmaf(l[i], w.y, w.x) : l[i];
+        acc[i][0] = in ? fmaf(w.y, acc[i][0], mul_rn(w.x, x0)) : acc[i][0];
+        if (TWO) acc[i][1] = in ? fmaf(w.y, acc[i][1], mul_rn(w.x, x1)) : acc[i][1];
+      }
+    });
+    __builtin_amdgcn_wave_barrier();
+  }
+#pragma unroll
+  for (int i = 0; i < RL; i++) {
+    const int r = g + i * G;
+    const long qi = w0 + r, bt = b * a.T + qi;
+    if (r >= R || qi > qlast) continue;
+    if (d < a.D) store_from_f32(a.out, a.dt, bt * a.ldo + h * a.D + d, acc[i][0] / l[i]);
+    if (two) store_from_f32(a.out, a.dt, bt * a.ldo + h * a.D + d + 64, acc[i][1] / l[i]);
+    if (!CACHED && d == 0) {
+      float mr = m[0];
+#pragma unroll
+      for (int q = 1; q < R; q++) mr = q == r ? m[q] : mr;
+      a.lse[bt * a.HQ + h] = mr + logf(l[i]);
     }
   }
 }
 
-__global__ __launch_bounds__(256) void k_attn_dq_rows(RowArgs a) {
-  const int lane = threadIdx.x & 63;
-  const long row = blockIdx.x * 4L + (threadIdx.x >> 6);
-  if (row >= a.B * a.T * a.HQ) return;
-  const long h = row % a.HQ, bt = row / a.HQ, pos = bt % a.T, b = bt / a.T;
-  const long kvh = h / (a.HQ / a.HK);
-  const float scale = 1.f / sqrtf((float)a.D);
-  float q[2], dy[2], acc[2] = {0.f, 0.f};
-  float dl = 0.f;
-  for (int i = 0; i < 2; i++) {
-    long d = lane + 64 * i;
-    q[i] = d < a.D ? load_as_f32(a.q, a.dt, bt * a.ldq + h * a.D + d) : 0.f;
-    dy[i] = d < a.D ? a.dout[bt * a.lddo + h * a.D + d] : 0.f;
-    float ov = d < a.D ? load_as_f32(a.o, a.dt, bt * a.ldo + h * a.D + d) : 0.f;
-    dl += dy[i] * ov;
-  }
-  dl = wave_sum(dl);
-  if (lane == 0) a.delta[row] = dl;
-  const float lse = a.lse[row];
-  long first = a.window > 0 ? (pos + 1 - a.window > 0 ? pos + 1 - a.window : 0) : 0;
-  for (long p = first; p <= pos; p++) {
-    long kr = b * a.T + p;
-    float s = 0.f, dp = 0.f, kv[2];
-    for (int i = 0; i < 2; i++) {
-      long d = lane + 64 * i;
-      kv[i] = d < a.D ? load_as_f32(a.k, a.dt, kr * a.ldk + kvh * a.D + d) : 0.f;
-      float vv = d < a.D ? load_as_f32(a.v, a.dt, kr * a.ldv + kvh * a.D + d) : 0.f;
-      s += q[i] * kv[i];
-      dp += dy[i] * vv;
-    }
-    s = wave_sum(s);
-    dp = wave_sum(dp);
-    float pr = expf(s * scale - lse);
-    float ds = pr * (dp - dl) * scale;
-    for (int i = 0; i < 2; i++) acc[i] += ds * kv[i];
-  }
-  inv_rope_store(a.dq + bt * a.lddq + h * a.D, a.rope, pos, a.D, lane, acc[0], acc[1]);
+// column d (and d + 64) of a gradient row with the inverse rotation: x and
+// its pair partner y (column d ^ 1)
+__device__ __forceinline__ float inv_rope(const float* rope, long pos, long D, int d, float x, float y) {
+  if (!rope) return x;
+  const float2 cs = *(const float2*)(rope + 2 * (pos * (D / 2) + (d >> 1)));
+  const float xc = mul_rn(x, cs.x), ys = mul_rn(y, cs.y);
+  return (d & 1) ? xc - ys : xc + ys;
 }
 
-__global__ __launch_bounds__(256) void k_attn_dkv_rows(RowArgs a) {
-  const int lane = threadIdx.x & 63;
-  const long row = blockIdx.x * 4L + (threadIdx.x >> 6);  // (b*T + pos)*HK + kvh
-  if (row >= a.B * a.T * a.HK) return;
-  const long kvh = row % a.HK, bt = row / a.HK, pos = bt % a.T, b = bt / a.T;
-  const long group = a.HQ / a.HK;
+// DKV false: the fixed rows are queries (q, dO), the streamed ones keys (k, v):
+// dQ and Delta.  DKV true: fixed keys (k, v), streamed queries (q, dO) of the
+// group's heads in turn: dK | dV.
+template <int C, int R, bool DKV>
+__global__ __launch_bounds__(256) void k_attn_bwd_rows(RowArgs a) {
+  constexpr int L = C < 64 ? C : 64, G = 64 / L, RL = (R + G - 1) / G, LD = C + 4;
+  constexpr bool TWO = C > 64;  // a second column per lane
+  extern __shared__ __attribute__((aligned(16))) float rt[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float *X = rt, *Y = X + RT_KEYS * LD, *A = Y + RT_KEYS * LD, *Bv = A + 4 * R * LD, *P = Bv + 4 * R * LD;
+  const long heads = DKV ? a.HK : a.HQ;
+  const long nblk = (a.T + 4 * R - 1) / (4 * R), per = heads * a.B, id = blockIdx.x;
+  // the longest walks first: the last queries, the first keys
+  const long blk = DKV ? id / per : nblk - 1 - id / per, h = (id % per) / a.B, b = id % a.B;
+  const long group = a.HQ / a.HK, f0 = blk * 4 * R, base = b * a.T, last = base + a.T - 1;
   const float scale = 1.f / sqrtf((float)a.D);
-  float k[2], v[2], ak[2] = {0.f, 0.f}, av[2] = {0.f, 0.f};
-  for (int i = 0; i < 2; i++) {
-    long d = lane + 64 * i;
-    k[i] = d < a.D ? load_as_f32(a.k, a.dt, bt * a.ldk + kvh * a.D + d) : 0.f;
-    v[i] = d < a.D ? load_as_f32(a.v, a.dt, bt * a.ldv + kvh * a.D + d) : 0.f;
-  }
-  long end = a.window > 0 ? (pos + a.window < a.T ? pos + a.window : a.T) : a.T;
-  for (long gi = 0; gi < group; gi++) {
-    long h = kvh * group + gi;
-    for (long qp = pos; qp < end; qp++) {
-      long qr = (b * a.T + qp);
-      float s = 0.f, dp = 0.f, qv[2], dy[2];
+  const size_t es = a.dt == SJ_BF16 ? 2 : 4;
+  const long kvh = DKV ? h : h / group;
+  const char *kh = (const char*)a.k + kvh * a.D * es, *vh = (const char*)a.v + kvh * a.D * es;
+  const bool kvec = rt_vec(kh, a.dt, a.ldk, a.D), vvec = rt_vec(vh, a.dt, a.ldv, a.D);
+  const long flast = (f0 + 4 * R < a.T ? f0 + 4 * R : a.T) - 1, w0 = f0 + wave * R;
+  float lse[R], dl[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) lse[r] = dl[r] = 0.f;
+  if constexpr (DKV) {
+    rt_stage<C>(A, 4 * R, kh, a.dt, a.ldk, base + f0, last, a.D, kvec);
+    rt_stage<C>(Bv, 4 * R, vh, a.dt, a.ldv, base + f0, last, a.D, vvec);
+  } else {
+    const char* qh = (const char*)a.q + h * a.D * es;
+    const float* dh = a.dout + h * a.D;
+    rt_stage<C>(A, 4 * R, qh, a.dt, a.ldq, base + f0, last, a.D, rt_vec(qh, a.dt, a.ldq, a.D));
+    rt_stage<C>(Bv, 4 * R, dh, SJ_F32, a.lddo, base + f0, last, a.D, rt_vec(dh, SJ_F32, a.lddo, a.D));
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const long bt = base + w0 + r;
+      if (w0 + r > flast) continue;
+      float t = 0.f;
       for (int i = 0; i < 2; i++) {
-        long d = lane + 64 * i;
-        qv[i] = d < a.D ? load_as_f32(a.q, a.dt, qr * a.ldq + h * a.D + d) : 0.f;
-        dy[i] = d < a.D ? a.dout[qr * a.lddo + h * a.D + d] : 0.f;
-        s += qv[i] * k[i];
-        dp += dy[i] * v[i];
+        const long c = lane + 64 * i;
+        if (c < a.D) t = fmaf(a.dout[bt * a.lddo + h * a.D + c], load_as_f32(a.o, a.dt, bt * a.ldo + h * a.D + c), t);
       }
-      s = wave_sum(s);
-      dp = wave_sum(dp);
-      long qrow = qr * a.HQ + h;
-      float pr = expf(s * scale - a.lse[qrow]);
-      float ds = pr * (dp - a.delta[qrow]) * scale;
-      for (int i = 0; i < 2; i++) {
-        ak[i] += ds * qv[i];
-        av[i] += pr * dy[i];
-      }
+      dl[r] = wave_sum(t);
+      lse[r] = a.lse[bt * a.HQ + h];
+      if (lane == 0) a.delta[bt * a.HQ + h] = dl[r];
     }
   }
-  inv_rope_store(a.dk + bt * a.lddk + kvh * a.D, a.rope, pos, a.D, lane, ak[0], ak[1]);
-  for (int i = 0; i < 2; i++) {
-    long d = lane + 64 * i;
-    if (d < a.D) a.dv[bt * a.lddv + kvh * a.D + d] = av[i];
+  const int d = lane & (L - 1), g = lane / L;
+  const bool two = TWO && d + 64 < a.D;
+  float acc1[RL][2], acc2[RL][2];
+#pragma unroll
+  for (int i = 0; i < RL; i++) acc1[i][0] = acc1[i][1] = acc2[i][0] = acc2[i][1] = 0.f;
+  const float *Aw = A + wave * R * LD, *Bw = Bv + wave * R * LD;
+  float2* Pw = (float2*)P + wave * R * RT_KEYS;  // (ds, probability) per fixed and streamed row
+  // visible streamed rows of a fixed row f: keys [lo, f], or queries [f, hi]
+  auto lo_of = [&](long f) { return DKV ? f : a.window > 0 && f + 1 > a.window ? f + 1 - a.window : 0L; };
+  auto hi_of = [&](long f) { return !DKV ? f : a.window > 0 && f + a.window < a.T ? f + a.window - 1 : a.T - 1; };
+  const long wl = w0 + R - 1 < flast ? w0 + R - 1 : flast;  // the wave's last row
+  for (long gi = 0; gi < (DKV ? group : 1); gi++) {
+    const long hq = kvh * group + gi;
+    const char* xs = DKV ? (const char*)a.q + hq * a.D * es : kh;
+    const void* ys = DKV ? (const void*)(a.dout + hq * a.D) : (const void*)vh;
+    const long xld = DKV ? a.ldq : a.ldk, yld = DKV ? a.lddo : a.ldv;
+    const int ydt = DKV ? (int)SJ_F32 : a.dt;
+    const bool xvec = DKV ? rt_vec(xs, a.dt, xld, a.D) : kvec, yvec = DKV ? rt_vec(ys, ydt, yld, a.D) : vvec;
+    for (long k0 = lo_of(f0); k0 <= hi_of(flast); k0 += RT_KEYS) {
+      const long p = k0 + lane;
+      __syncthreads();
+      rt_stage<C>(X, RT_KEYS, xs, a.dt, xld, base + k0, last, a.D, xvec);
+      rt_stage<C>(Y, RT_KEYS, ys, ydt, yld, base + k0, last, a.D, yvec);
+      float lj = 0.f, dj = 0.f;
+      if (DKV && p < a.T) {
+        lj = a.lse[(base + p) * a.HQ + hq];
+        dj = a.delta[(base + p) * a.HQ + hq];
+      }
+      __syncthreads();
+      if (w0 > flast || k0 > hi_of(wl) || k0 + RT_KEYS <= lo_of(w0)) continue;  // nothing visible to this wave
+      float s[R], dp[R];
+      rt_dots<C, R>(Aw, X + lane * LD, s);
+      rt_dots<C, R>(Bw, Y + lane * LD, dp);
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const float pr = expf(fmaf(scale, s[r], -(DKV ? lj : lse[r])));
+        Pw[r * RT_KEYS + lane] = make_float2(mul_rn(mul_rn(pr, dp[r] - (DKV ? dj : dl[r])), scale), pr);
+      }
+      __builtin_amdgcn_wave_barrier();
+      // this lane's fixed rows' visible rows of the tile
+      const float2* Pl[RL];
+      int lo[RL], hi[RL];
+#pragma unroll
+      for (int i = 0; i < RL; i++) {
+        const int r = g + i * G < R ? g + i * G : R - 1;
+        const long l0 = lo_of(w0 + r) - k0, h0 = hi_of(w0 + r) - k0;
+        Pl[i] = Pw + r * RT_KEYS;
+        lo[i] = l0 > 0 ? (int)(l0 < RT_KEYS ? l0 : RT_KEYS) : 0;
+        hi[i] = h0 < RT_KEYS ? (int)h0 : RT_KEYS;
+      }
+      rt_walk(lo_of(w0) - k0, lo_of(wl) - k0, hi_of(w0) - k0, hi_of(wl) - k0, [&](int j, bool masked) {
+        const float x0 = X[j * LD + d], x1 = TWO ? X[j * LD + d + 64] : 0.f;
+        const float y0 = DKV ? Y[j * LD + d] : 0.f, y1 = DKV && TWO ? Y[j * LD + d + 64] : 0.f;
+#pragma unroll
+        for (int i = 0; i < RL; i++) {
+          const float2 w = Pl[i][j];
+          const bool in = !masked || (j >= lo[i] && j <= hi[i]);
+          acc1[i][0] = in ? fmaf(w.x, x0, acc1[i][0]) : acc1[i][0];
+          if (TWO) acc1[i][1] = in ? fmaf(w.x, x1, acc1[i][1]) : acc1[i][1];
+          if (DKV) acc2[i][0] = in ? fmaf(w.y, y0, acc2[i][0]) : acc2[i][0];
+          if (DKV && TWO) acc2[i][1] = in ? fmaf(w.y, y1, acc2[i][1]) : acc2[i][1];
+        }
+      });
+      __builtin_amdgcn_wave_barrier();
+    }
   }
+#pragma unroll
+  for (int i = 0; i < RL; i++) {
+    const float p0 = __shfl_xor(acc1[i][0], 1, 64), p1 = __shfl_xor(acc1[i][1], 1, 64);
+    const int r = g + i * G;
+    const long f = w0 + r, bt = base + f;
+    if (r >= R || f > flast) continue;
+    float* dst = DKV ? a.dk + bt * a.lddk + h * a.D : a.dq + bt * a.lddq + h * a.D;
+    if (d < a.D) dst[d] = inv_rope(a.rope, f, a.D, d, acc1[i][0], p0);
+    if (two) dst[d + 64] = inv_rope(a.rope, f, a.D, d + 64, acc1[i][1], p1);
+    if (DKV) {
+      float* dv = a.dv + bt * a.lddv + h * a.D;
+      if (d < a.D) dv[d] = acc2[i][0];
+      if (two) dv[d + 64] = acc2[i][1];
+    }
+  }
+}
+
+// Rows per wave: 4 once that gives two workgroups per CU (a staged row then
+// serves 16 fixed ones); below, as many as fill the lanes with columns
+// (shorter chains, more workgroups).
+inline int rt_cols(long D) { return D <= 4 ? 4 : D <= 8 ? 8 : D <= 16 ? 16 : D <= 32 ? 32 : D <= 64 ? 64 : 128; }
+inline int rt_rows(long D, long rows_heads) {
+  const int C = rt_cols(D);
+  return C <= 16 || rows_heads / 16 >= 512 ? 4 : C == 32 ? 2 : 1;
+}
+
+typedef void (*rt_kernel)(RowArgs);
+template <int C, int R> struct RtFwd { static constexpr rt_kernel fn = k_attn_fwd_rows<C, R, false>; static constexpr int bwd = 0; };
+template <int C, int R> struct RtCached { static constexpr rt_kernel fn = k_attn_fwd_rows<C, R, true>; static constexpr int bwd = 0; };
+template <int C, int R> struct RtDq { static constexpr rt_kernel fn = k_attn_bwd_rows<C, R, false>; static constexpr int bwd = 1; };
+template <int C, int R> struct RtDkv { static constexpr rt_kernel fn = k_attn_bwd_rows<C, R, true>; static constexpr int bwd = 1; };
+
+// f(kernel, rows per wave, LDS bytes) for the instantiation that serves
+// head_dim D and `rows_heads` fixed rows over all heads
+template <template <int, int> class K, class F>
+void rt_pick(long D, long rows_heads, F f) {
+  const int C = rt_cols(D), R = rt_rows(D, rows_heads);
+#define SJ_RT(c, r) \
+  if (C == c && R == r) return f(K<c, r>::fn, r, rt_lds_bytes<c, r>(K<c, r>::bwd))
+  SJ_RT(4, 4);
+  SJ_RT(8, 4);
+  SJ_RT(16, 4);
+  SJ_RT(32, 2);
+  SJ_RT(32, 4);
+  SJ_RT(64, 1);
+  SJ_RT(64, 4);
+  SJ_RT(128, 1);
+  SJ_RT(128, 4);
+#undef SJ_RT
+}
+template <template <int, int> class K>
+void launch_rows(hipStream_t s, const RowArgs& a, long heads) {
+  rt_pick<K>(a.D, a.B * a.T * heads, [&](rt_kernel k, int R, size_t lds) {
+    const long grid = (a.T + 4 * R - 1) / (4 * R) * heads * a.B;
+    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(256), lds, s, a);
+  });
+}
+
+// Raise the dynamic-LDS limit of the kernels that stage more than 64 KB
+// (head_dim above 64) once, outside any capture.
+int rows_prepare() {
+  static int done = 0, status = SJ_OK;
+  if (done) return status;
+  done = 1;
+  auto set = [&](rt_kernel k, int, size_t lds) {
+    if (status) return;
+    const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) status = sjh::hip_check(e, "attention rows: LDS attribute");
+  };
+  for (long rows : {1L, 1L << 20}) {
+    rt_pick<RtFwd>(128, rows, set);
+    rt_pick<RtCached>(128, rows, set);
+    rt_pick<RtDq>(128, rows, set);
+    rt_pick<RtDkv>(128, rows, set);
+  }
+  return status;
 }
 
 bool use_mfma(int dtype, long head_dim, long window, long t, long ldq, long ldk, long ldv, long ldo,
@@ -1132,8 +1401,8 @@ extern "C" int sj_attention_fwd(void* stream, const void* q, long ldq, const voi
     a.q = q; a.k = k; a.v = v; a.ldq = ldq; a.ldk = ldk; a.ldv = ldv; a.ldo = ldo;
     a.out = o; a.lse = lse; a.dt = dtype; a.B = batch; a.T = t; a.HQ = hq; a.HK = hk; a.D = head_dim;
     a.window = window;
-    long rows = batch * t * hq;
-    hipLaunchKernelGGL(k_attn_fwd_rows<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, a);
+    if (int st = rows_prepare()) return st;
+    launch_rows<RtFwd>(s, a, hq);
   }
   SJ_LAUNCH_CHECK("hierarchy_attention");
   return SJ_OK;
@@ -1159,8 +1428,8 @@ extern "C" int sj_attention_fwd_cached(void* stream, const void* q, long ldq, co
   a.q = q; a.k = k; a.v = v; a.ldq = ldq; a.ldk = ldkv; a.ldv = ldkv; a.ldo = ldo;
   a.out = o; a.dt = dtype; a.B = 1; a.T = tq; a.HQ = hq; a.HK = hk; a.D = head_dim;
   a.window = window; a.offset = offset;
-  long rows = tq * hq;
-  hipLaunchKernelGGL(k_attn_fwd_rows<true>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, a);
+  if (int st = rows_prepare()) return st;
+  launch_rows<RtCached>(s, a, hq);
   SJ_LAUNCH_CHECK("hierarchy_attention (cached)");
   return SJ_OK;
 }
@@ -1197,17 +1466,16 @@ extern "C" int sj_attention_bwd(void* stream, const void* q, long ldq, const voi
     a.dq = dq; a.dk = dk; a.dv = dv; a.delta = delta; a.lddq = lddq; a.lddk = lddk; a.lddv = lddv;
     a.dt = dtype; a.B = batch; a.T = t; a.HQ = hq; a.HK = hk; a.D = head_dim; a.window = window;
     a.rope = rope_table;
-    long rows = batch * t * hq;
-    hipLaunchKernelGGL(k_attn_dq_rows, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, a);
-    long krows = batch * t * hk;
-    hipLaunchKernelGGL(k_attn_dkv_rows, dim3((unsigned)((krows + 3) / 4)), dim3(256), 0, s, a);
+    if (int st = rows_prepare()) return st;
+    launch_rows<RtDq>(s, a, hq);
+    launch_rows<RtDkv>(s, a, hk);
   }
   SJ_LAUNCH_CHECK("hierarchy_attention_backward");
   return SJ_OK;
 }
 
 namespace sjh {
-int attention_prepare() { return SJ_OK; }
+int attention_prepare() { return rows_prepare(); }
 }  // namespace sjh
 
 extern "C" int sj_attention_fwd_t(void* stream, const uint16_t* q, long ldq, const uint16_t* k, long ldk,

@@ -177,6 +177,21 @@ int qkv_fwd_t_out(void* stream, const uint16_t* x, long ldx, long M, long D, con
 // cached grouped attention on the MFMA layout (bf16, head_dim 64), one sequence
 int attention_fwd_cached_t(void* stream, const uint16_t* q, long ldq, const uint16_t* k, const uint16_t* v, long ldkv,
                            long capacity, long tq, long offset, long hq, long hk, long window, uint16_t* o, long ldo);
+// The cached path's products for up to DECODE_ROWS rows (decode.hip): RMSNorm +
+// project_qkv + RoPE (rows from x, or the embedding rows of the host's ids,
+// then also written to xout), projection + residual, RMSNorm + gate/up +
+// SwiGLU (h only), final RMSNorm + head on one row; the bits of the tiled ones
+constexpr int DECODE_ROWS = 16;
+bool decode_rows_ok(long n, long d);
+int decode_qkv(hipStream_t s, const uint16_t* x, const uint16_t* table, const int32_t* ids, uint16_t* xout,
+               const uint16_t* wn, float eps, long n, long d, const uint16_t* wqkv_t, long kv, uint16_t* q, uint16_t* k,
+               uint16_t* v, const float* rope, long head_dim);
+int decode_residual(hipStream_t s, const uint16_t* a, long n, long K, const uint16_t* w_t, long N, const uint16_t* r,
+                    uint16_t* y);
+int decode_gate_up(hipStream_t s, const uint16_t* x, const uint16_t* wn, float eps, long n, long d, const uint16_t* wg_t,
+                   const uint16_t* wu_t, long F, uint16_t* h);
+int decode_head(hipStream_t s, const uint16_t* x, const uint16_t* wn, float eps, long d, const uint16_t* w_hi,
+                const uint16_t* w_lo, long N, float* logits, float* logits2);
 int attention_kv_reduce(hipStream_t s, const float* part, long group, long M, long T, long N, long KV,
                         const float* rope, uint16_t* g_hi, uint16_t* g_lo, long ldg, uint16_t* gt_hi, uint16_t* gt_lo,
                         long ldgt);

@@ -2904,8 +2904,12 @@ int calloc_(sj_cache* c, void** p, size_t bytes) {
 // cached_blocks (architecture.rs:474-533): the blocks of stage si over n
 // new rows in c->x[0] at positions L .. L + n - 1 of the stage's cache;
 // then the stage's closing norm into `out` (the encoder, global or decoder
-// norm, or the final norm of a one-stage model)
-int cached_blocks(sj_model* m, sj_cache* c, int si, long n, long L, void* out) {
+// norm, or the final norm of a one-stage model; null: *last receives the
+// blocks' output rows instead).  Up to 16 rows run the few-row products
+// (decode.hip); `tokens` (host, nullable, few rows only): the first layer's
+// rows are these tokens' embeddings, not c->x[0].
+int cached_blocks(sj_model* m, sj_cache* c, int si, long n, long L, void* out, const int32_t* tokens = nullptr,
+                  void** last = nullptr) {
   const Stage& S = m->stages[si];
   hipStream_t s = m->stream;
   const long d = S.d, J = S.J, F = S.F, cap = c->scap[si];
@@ -2921,8 +2925,27 @@ int cached_blocks(sj_model* m, sj_cache* c, int si, long n, long L, void* out) {
     void* xo = c->x[cur ^ 1];
     char* kc = (char*)c->keys[l] + L * J * es;
     char* vc = (char*)c->values[l] + L * J * es;
+    const bool few = m->planes && sjh::decode_rows_ok(n, d);
+    if (few) {
+      const uint16_t *W = m->mirror, *WT = m->mirror_t;
+      const bool emb = tokens && l == S.first;
+      TRY(sjh::decode_qkv(s, emb ? nullptr : (const uint16_t*)x, emb ? W + m->emb : nullptr, emb ? tokens : nullptr,
+                          emb ? (uint16_t*)x : nullptr, W + y.an, eps, n, d, WT + y.qkv, J, (uint16_t*)c->q,
+                          (uint16_t*)kc, (uint16_t*)vc, rope, S.Dh));
+      TRY(sj_attention_fwd_cached(s, c->q, d, c->keys[l], c->values[l], J, cap, dt, n, L, S.HQ, S.HK, S.Dh, S.window,
+                                  c->o, d));
+      TRY(sjh::decode_residual(s, (const uint16_t*)c->o, n, d, WT + y.wo, d, (const uint16_t*)x, (uint16_t*)c->x1));
+      if (!m->E) {
+        TRY(sjh::decode_gate_up(s, (const uint16_t*)c->x1, W + y.fn, eps, n, d, WT + y.gu, WT + y.gu + F * d, F,
+                                (uint16_t*)c->hh));
+        TRY(sjh::decode_residual(s, (const uint16_t*)c->hh, n, F, WT + y.down, d, (const uint16_t*)c->x1, (uint16_t*)xo));
+        cur ^= 1;
+        continue;
+      }
+    }
     if (m->planes) {
       const uint16_t *W = m->mirror, *WT = m->mirror_t;
+      if (!few) {
       TRY(sj_rmsnorm_fwd_t(s, (const uint16_t*)x, W + y.an, (uint16_t*)c->z, nullptr, 0, n, d, eps));
       TRY(sjh::qkv_fwd_t_out(s, (const uint16_t*)c->z, d, n, d, WT + y.qkv, d, d, J, (uint16_t*)c->q, d,
                              (uint16_t*)kc, J, (uint16_t*)vc, J, rope, rope_t, S.Dh, nullptr, 0));
@@ -2930,6 +2953,7 @@ int cached_blocks(sj_model* m, sj_cache* c, int si, long n, long L, void* out) {
                                   c->o, d));
       TRY(sj_linear_residual_fwd_t(s, (const uint16_t*)c->o, d, n, d, WT + y.wo, d, d, (const uint16_t*)x, d,
                                    (uint16_t*)c->x1, d));
+      }
       TRY(sj_rmsnorm_fwd_t(s, (const uint16_t*)c->x1, W + y.fn, (uint16_t*)c->z2, nullptr, 0, n, d, eps));
       if (m->E) {  // routed experts over the new rows (architecture.rs:516-529)
         const long E = m->E, K = m->K, mc = sj_route_pack_capacity(n * K, E);
@@ -2963,7 +2987,8 @@ int cached_blocks(sj_model* m, sj_cache* c, int si, long n, long L, void* out) {
     }
     cur ^= 1;
   }
-  TRY(sj_rmsnorm_fwd(s, c->x[cur], dt, wc(m, S.norm), dt, out, n, d, eps));
+  if (last) *last = c->x[cur];
+  if (out) TRY(sj_rmsnorm_fwd(s, c->x[cur], dt, wc(m, S.norm), dt, out, n, d, eps));
   return SJ_OK;
 }
 
@@ -3170,6 +3195,16 @@ extern "C" int sj_model_forward_cached(sj_model* m, sj_cache* c, const int32_t* 
   const long d = m->d;
   const int dt = m->dt;
   if (m->mt_stale) TRY(transpose_mirror(m));  // weights updated since the last forward
+  if (m->lm_planes && !m->hier && sjh::decode_rows_ok(n, d)) {
+    // few rows: the tokens travel as kernel arguments, the final norm and the
+    // head run on the last row in one launch, which writes `logits` itself
+    void* x = nullptr;
+    TRY(cached_blocks(m, c, 0, n, c->length, nullptr, tokens, &x));
+    TRY(sjh::decode_head(s, (const uint16_t*)x + (n - 1) * d, m->mirror + m->final_norm, m->c.norm_epsilon, d, m->hp[2],
+                         m->hp[3], m->HV, c->logits, logits));
+    c->length += n;
+    return SJ_OK;
+  }
   SJ_HIP(hipMemcpyAsync(c->ids, tokens, (size_t)n * 4, hipMemcpyHostToDevice, s));
   long row = n - 1;  // the row of c->hn that holds the last token's output
   if (m->hier) {

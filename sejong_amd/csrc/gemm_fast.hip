@@ -258,8 +258,8 @@ constexpr size_t lds_bytes() {
 template <int BM, int BN, int PA, int PB, int EPI, int NS, int TM = 0>
 __global__ __launch_bounds__(NT) void k_gemm_fast(FParams p) {
   constexpr bool TA = (TM & 1) != 0, TB = (TM & 2) != 0;
-  static_assert(!(TA || TB) || ((EPI == E_STORE || EPI == E_PARTIAL) && BM % 64 == 0 && BN % 64 == 0),
-                "row-layout operands: plain products with 64-multiple tiles");
+  static_assert(!(TA || TB) || EPI == E_STORE || EPI == E_PARTIAL, "row-layout operands: plain products");
+  static_assert((!TA || BM % 64 == 0) && (!TB || BN % 64 == 0), "row-layout operands: 64-column sub-tiles");
   constexpr bool DUAL = EPI == E_GATEUP;
   constexpr int NBM = DUAL ? 2 : 1;
   constexpr int WM = BM / 2, WN = BN / 2, MB = WM / 16, NB = WN / 16;
@@ -1397,6 +1397,59 @@ bool plan_kw(long M, long N, long K, int pa, int& splits) {
   return true;
 }
 
+// Tiles of the parameter VJP's coefficient product (C = A Y, both operands
+// hi/lo planes, Y in row layout, few rows of A against long K).  It is bound
+// by the LDS DMA: a 64 x 64 tile stages 2 x (64 + 64) rows for 3 x 64 x 64
+// products and Y once per row tile.  A tile over all the rows (96, 160 or
+// 192) and 64 or 128 columns stages both less often; what a CU then moves was
+// about 55 KB/us with two workgroups resident and 43 with one.  The plan takes
+// the tile and the K slices (at most the general plan's: the workspace holds
+// those) with the least modelled time: rounds of workgroups, each K / slices
+// stages, and the partials' write and read.  144 x 5504 x 16384: 155 (64 x 64)
+// -> 107 us; 64-row tiles stay with the general plan.
+bool plan_tall(long M, long N, long K, int& bm, int& bn, int& splits) {
+  if (K < 8192 || M > 512) return false;
+  const long cu = cus();
+  double best = 0;
+  int bs = 1, bbm = 0, bbn = 0;
+  for (int cn : {64, 128})
+    for (int cm : {64, 96, 128, 160, 192}) {
+      const long t = tiles(M, N, cm, cn);
+      const double stage = 0.25 * (cm + cn);  // KB: 2 (cm + cn) rows of 128 bytes
+      const int occ = 4 * stage <= 160 ? 2 : 1;
+      const double per = (double)occ * stage / (occ == 2 ? 55.0 : 43.0);  // us a stage
+      for (int s = 1; s <= splits; s++) {
+        const double c = (double)((t * s + cu * occ - 1) / (cu * occ)) * ((double)K / 64 / s) * per +
+                         (s > 1 ? s * (double)M * (double)N * 8.0 / 4.5e6 : 0.0);
+        if (best == 0 || c < best) {
+          best = c;
+          bs = s;
+          bbm = cm;
+          bbn = cn;
+        }
+      }
+    }
+  if (bbm == 64) return false;
+  bm = bbm;
+  bn = bbn;
+  splits = bs;
+  return true;
+}
+
+template <int EPI>
+int launch_tall(hipStream_t s, const FParams& p, int bm, int bn, int splits) {
+  if (bn == 64) {
+    if (bm == 96) return launch<96, 64, 2, 2, EPI, 2>(s, p, splits);
+    if (bm == 128) return launch<128, 64, 2, 2, EPI, 2>(s, p, splits);
+    if (bm == 160) return launch<160, 64, 2, 2, EPI, 2>(s, p, splits);
+    return launch<192, 64, 2, 2, EPI, 2>(s, p, splits);
+  }
+  if (bm == 96) return launch<96, 128, 2, 2, EPI, 2>(s, p, splits);
+  if (bm == 128) return launch<128, 128, 2, 2, EPI, 2>(s, p, splits);
+  if (bm == 160) return launch<160, 128, 2, 2, EPI, 2>(s, p, splits);
+  return launch<192, 128, 2, 2, EPI, 2>(s, p, splits);
+}
+
 template <int EPI, int PA, int PB, int TM = 0>
 int launch_tile(hipStream_t s, const FParams& p, int bm, int bn, int splits) {
   // both operands split: a 128x128 stage does not fit three deep in LDS
@@ -1475,6 +1528,17 @@ int set_attrs_tiles() {
   if (!s) s = set_attr<64, 64, PA, PB, EPI, TM>();
   return s;
 }
+template <int EPI>
+int set_attrs_tall() {
+  int s = set_attr<96, 64, 2, 2, EPI, 2>();
+  if (!s) s = set_attr<160, 64, 2, 2, EPI, 2>();
+  if (!s) s = set_attr<192, 64, 2, 2, EPI, 2>();
+  if (!s) s = set_attr<96, 128, 2, 2, EPI, 2>();
+  if (!s) s = set_attr<128, 128, 2, 2, EPI, 2>();
+  if (!s) s = set_attr<160, 128, 2, 2, EPI, 2>();
+  if (!s) s = set_attr<192, 128, 2, 2, EPI, 2>();
+  return s;
+}
 template <int EPI, int TM = 0>
 int set_attrs_planes() {
   int s = SJ_OK;
@@ -1521,6 +1585,8 @@ int gemm_fast_prepare() {
   if (!status) status = set_attrs_tiles<E_PARTIAL, 1, 2, 1>();
   if (!status) status = set_attrs_tiles<E_STORE, 2, 2, 2>();
   if (!status) status = set_attrs_tiles<E_PARTIAL, 2, 2, 2>();
+  if (!status) status = set_attrs_tall<E_STORE>();
+  if (!status) status = set_attrs_tall<E_PARTIAL>();
   if (!status) status = set_attrs_kw<E_STORE>();
   if (!status) status = set_attrs_kw<E_PARTIAL>();
   return status;
@@ -1602,6 +1668,8 @@ int gemm_planes(void* stream, long M, long N, long K, const uint16_t* a_hi, cons
   if constexpr (TM == 3)
     if (plan_kw(M, N, K, pa, splits)) return gemm_kw(s, p, pb, splits, workspace, workspace_bytes);
   plan(M, N, K, pa, bm, bn, splits, TM != 0);
+  bool tall = false;
+  if constexpr (TM == 2) tall = plan_tall(M, N, K, bm, bn, splits);
   if (splits > 1 && workspace && workspace_bytes >= sizeof(float) * (size_t)splits * M * N) {
     long kchunk = (K + splits - 1) / splits;
     kchunk = (kchunk + BK - 1) / BK * BK;
@@ -1609,7 +1677,9 @@ int gemm_planes(void* stream, long M, long N, long K, const uint16_t* a_hi, cons
     p.kchunk = kchunk;
     p.partial = (float*)workspace;
     int st;
-    if constexpr (TM == 1 || TM == 2)
+    if (tall)
+      st = launch_tall<E_PARTIAL>(s, p, bm, bn, splits);
+    else if constexpr (TM == 1 || TM == 2)
       st = launch_planes_one<E_PARTIAL, TM>(s, p, pa, pb, bm, bn, splits);
     else
       st = launch_planes<E_PARTIAL, TM>(s, p, pa, pb, bm, bn, splits);
@@ -1617,7 +1687,9 @@ int gemm_planes(void* stream, long M, long N, long K, const uint16_t* a_hi, cons
     reduce_partials(s, p, splits, workspace);
   } else {
     int st;
-    if constexpr (TM == 1 || TM == 2)
+    if (tall)
+      st = launch_tall<E_STORE>(s, p, bm, bn, 1);
+    else if constexpr (TM == 1 || TM == 2)
       st = launch_planes_one<E_STORE, TM>(s, p, pa, pb, bm, bn, 1);
     else
       st = launch_planes<E_STORE, TM>(s, p, pa, pb, bm, bn, 1);

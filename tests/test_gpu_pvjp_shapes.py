@@ -1,0 +1,89 @@
+"""The parameter VJP's kernels at the edges of their ranges: ranks 1, 16, 17,
+32, 33 and 64, ragged rows, more than 64 selected blocks (the serial draws),
+and the coefficient product's row tiles (64, 96, 128, 160, 192 rows)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from oracle import pvjp as P
+from tests.gpu_util import dev, empty, rel, rnd, sync, zeros
+
+pytestmark = pytest.mark.gpu
+cf = ctypes.c_float
+
+
+@pytest.fixture(scope="module")
+def N():
+    from sejong_amd import _native as N
+    N.load()
+    return N
+
+
+@pytest.mark.parametrize("A,B,block,S,R,seed", [
+    (1024, 2752, 32, 4, 16, 7), (1000, 300, 32, 32, 64, 1 << 40), (37, 5, 8, 5, 5, 3), (64, 64, 1, 64, 64, 11),
+    (260, 70, 2, 100, 16, 5),   # more than 64 blocks
+    (64, 200, 16, 2, 100, 9),   # more than 64 columns
+    (64, 1, 64, 1, 1, 2 ** 64 - 1),
+])
+def test_indices_match_the_reference_draws(N, A, B, block, S, R, seed):
+    NB = -(-A // block)
+    scr, cols, rows, fmap = zeros(B + NB, "i32"), zeros(R, "i32"), zeros(S * block, "i32"), zeros(A, "i32")
+    N.api.sj_pvjp_indices(None, ctypes.c_uint64(seed), A, B, NB, S, R, block, scr.p, cols.p, rows.p, fmap.p)
+    sync()
+    c, r, m = P.indices(seed, A, B, NB, S, R, block)
+    np.testing.assert_array_equal(cols.host(), c)
+    np.testing.assert_array_equal(rows.host(), r)
+    np.testing.assert_array_equal(fmap.host(), m)
+
+
+@pytest.mark.parametrize("n,R,dt,dup", [(64, 1, "f32", False), (65, 16, "bf16", False), (1000, 17, "f32", False),
+                                        (16400, 32, "bf16", False), (777, 33, "f32", True), (2048, 64, "bf16", True)])
+def test_basis_orthonormal_span_and_drop(N, n, R, dt, dup):
+    """Q^T Q = I on the kept columns, Q spans the picked columns, a duplicated
+    column becomes zero (n x R sums of fp32-rounded Q: 1e-6)."""
+    rng = np.random.default_rng(n + R)
+    B = R + 9
+    y = rnd((n, B), dt, rng)
+    cols = rng.permutation(B)[:R].astype(np.int32)
+    if dup:
+        cols[R - 1] = cols[0]
+    q = empty(n * R)
+    lib = N.load()
+    wb = lib.sj_pvjp_basis_workspace_bytes(n, R)
+    ws = empty(wb, "u8")
+    N.api.sj_pvjp_basis(None, dev(y, dt).p, 4 if dt == "bf16" else 0, B, n, dev(cols, "i32").p, R,
+                        cf(lib.sj_pvjp_basis_tolerance(n, R)), q.p, ws.p, wb)
+    sync()
+    Q = q.host().reshape(n, R)
+    keep = R - 1 if dup else R
+    if dup:
+        assert np.all(Q[:, R - 1] == 0)
+    assert np.max(np.abs(Q[:, :keep].T @ Q[:, :keep] - np.eye(keep))) < 2e-6
+    V = y[:, cols[:keep]]
+    Qr, _ = np.linalg.qr(V)
+    assert rel(Q[:, :keep] @ (Q[:, :keep].T @ V), Qr @ (Qr.T @ V)) < 2e-6
+
+
+@pytest.mark.parametrize("rows,b,n", [(48, 200, 8192), (80, 136, 8200), (112, 64, 8192), (144, 264, 8256),
+                                      (176, 72, 16384), (272, 320, 8192), (145, 8, 9000)])
+def test_coefficient_tiles(N, rows, b, n):
+    """E dY with both operands as hi/lo planes, dY in row layout: against FP64
+    (three bf16 products of four: 2^-16 per term, random signs)."""
+    rng = np.random.default_rng(rows + b)
+    split = lambda x: (O.round_to(x, "bf16"), O.round_to(x - O.round_to(x, "bf16"), "bf16"))
+    e = rng.normal(0, 1, (rows, n)).astype(np.float32).astype(np.float64)
+    dy = rng.normal(0, 1, (n, b)).astype(np.float32).astype(np.float64)
+    eh, el = split(e)
+    dh, dl = split(dy)
+    lib = N.load()
+    wb = lib.sj_pvjp_vjp_workspace_bytes(rows, b, n)
+    E = [dev(x, "bf16") for x in (eh, el)]
+    D = [dev(x, "bf16") for x in (dh, dl)]
+    for ws_bytes in (wb, 0):   # with and without room for K slices
+        C, ws = zeros(rows * b), empty(max(wb, 256), "u8")
+        N.api.sj_pvjp_vjp_rows(None, E[0].p, E[1].p, n, rows, n, D[0].p, D[1].p, b, b, C.p, b,
+                               ws.p if ws_bytes else None, ws_bytes)
+        sync()
+        assert rel(C.host(), (eh + el) @ (dh + dl)) < 3e-5

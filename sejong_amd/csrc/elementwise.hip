@@ -438,28 +438,49 @@ extern "C" int sj_embedding_fwd(void* stream, const void* w, int wd, const int32
 
 extern "C" size_t sj_embedding_bwd_workspace_bytes(long n, long vocab) { return 0; }
 
-// Faster form for d % 4 == 0, d <= 2048: each round scans 16 ids per thread
-// (4096 tokens), compacts the matches in token order with one block scan,
-// then every thread adds up to two float4 columns of the matching rows in
-// that order (the same order, hence the same bits, as k_embedding_bwd).
-constexpr int EMB_IDS = 16;
-// sq (nullable): FP64 sum of squares of the row this workgroup stores, at
-// sq[blockIdx.x] (the gradient-norm hook)
+// Faster form for d % 4 == 0 (16-byte rows): workgroup (v, c) owns columns
+// 128 c .. + 127 of vocabulary row v.  Each round scans 16 ids per thread
+// (4096 tokens) and compacts the matches in token order with one block scan;
+// then the matching rows come in batches of 64, eight 16-byte loads per
+// thread in flight into LDS while the batch before is added, column by
+// column in token order (the same order, hence the same bits, as
+// k_embedding_bwd).  Bound by the longest row of a skewed batch: one load in
+// flight per thread and column took 31 us with 256 of 4096 tokens alike (d
+// 384), now 10.
+constexpr int EMB_IDS = 16, EMB_COLS = 128, EMB_BATCH = 64;
+// sq (nullable): FP64 sum of squares of the columns this workgroup stores, at
+// sq[its linear index] (the gradient-norm hook)
 __global__ __launch_bounds__(EMB_THREADS) void k_embedding_bwd4(const float* __restrict__ dy,
                                                                 const int32_t* __restrict__ ids,
                                                                 float* __restrict__ dw, long n, long d, double* sq) {
-  __shared__ int matches[EMB_THREADS * EMB_IDS];
+  constexpr int W = EMB_THREADS * EMB_IDS, SLOTS = EMB_THREADS / (EMB_COLS / 4), PER = EMB_BATCH / SLOTS;
+  __shared__ uint16_t matches[W];
   __shared__ int wave_total[EMB_THREADS / 64];
+  __shared__ __attribute__((aligned(16))) float rows[EMB_BATCH * EMB_COLS];
   const int v = blockIdx.x;
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const long d4 = d >> 2;
-  float4 acc[2] = {make_float4(0.f, 0.f, 0.f, 0.f), make_float4(0.f, 0.f, 0.f, 0.f)};
-  for (long base = 0; base < n; base += (long)EMB_THREADS * EMB_IDS) {
+  const long col0 = (long)blockIdx.y * EMB_COLS;
+  // loading: 16-byte chunk lc of batch rows slot, slot + SLOTS, ...; adding: column t of the chunk
+  const int lc = t % (EMB_COLS / 4), slot = t / (EMB_COLS / 4);
+  const bool lok = col0 + 4 * lc < d, aok = t < EMB_COLS && col0 + t < d;
+  const float* src = dy + col0 + 4 * lc;
+  const bool ivec = ((uintptr_t)ids & 15) == 0;
+  float acc = 0.f;
+  for (long base = 0; base < n; base += W) {
     const long i0 = base + (long)t * EMB_IDS;
     uint32_t hit = 0;
+    if (ivec && i0 + EMB_IDS <= n) {
 #pragma unroll
-    for (int k = 0; k < EMB_IDS; k++)
-      if (i0 + k < n && ids[i0 + k] == v) hit |= 1u << k;
+      for (int k = 0; k < EMB_IDS; k += 4) {
+        const int4 q = *(const int4*)(ids + i0 + k);
+        hit |= (uint32_t)(q.x == v) << k | (uint32_t)(q.y == v) << (k + 1) | (uint32_t)(q.z == v) << (k + 2) |
+               (uint32_t)(q.w == v) << (k + 3);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < EMB_IDS; k++)
+        if (i0 + k < n && ids[i0 + k] == v) hit |= 1u << k;
+    }
     const int cnt = __popc(hit);
     int incl = cnt;  // inclusive scan over the wave
 #pragma unroll
@@ -479,36 +500,37 @@ __global__ __launch_bounds__(EMB_THREADS) void k_embedding_bwd4(const float* __r
     while (hit) {
       const int k = __ffs(hit) - 1;
       hit &= hit - 1;
-      matches[pos++] = (int)(i0 + k);
+      matches[pos++] = (uint16_t)(t * EMB_IDS + k);
     }
     __syncthreads();
+    float4 r[PER];
+    auto load = [&](int m0) {
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
-      const long col = t + (long)c * EMB_THREADS;
-      if (col < d4) {
-        const float4* src = (const float4*)dy + col;
-        for (int m = 0; m < total; m++) {
-          const float4 r = src[(long)matches[m] * d4];
-          acc[c].x += r.x; acc[c].y += r.y; acc[c].z += r.z; acc[c].w += r.w;
-        }
+      for (int i = 0; i < PER; i++) {
+        const int m = m0 + slot + SLOTS * i;
+        r[i] = lok && m < total ? *(const float4*)(src + (base + matches[m]) * d) : make_float4(0.f, 0.f, 0.f, 0.f);
       }
+    };
+    if (total > 0) load(0);
+    for (int m0 = 0; m0 < total; m0 += EMB_BATCH) {
+#pragma unroll
+      for (int i = 0; i < PER; i++) *(float4*)(rows + (slot + SLOTS * i) * EMB_COLS + 4 * lc) = r[i];
+      __syncthreads();
+      if (m0 + EMB_BATCH < total) load(m0 + EMB_BATCH);
+      if (aok) {
+        const int cntb = total - m0 < EMB_BATCH ? total - m0 : EMB_BATCH;
+#pragma unroll 8
+        for (int m = 0; m < cntb; m++) acc += rows[m * EMB_COLS + t];
+      }
+      __syncthreads();
     }
     __syncthreads();
   }
-  double q = 0.0;
-#pragma unroll
-  for (int c = 0; c < 2; c++) {
-    const long col = t + (long)c * EMB_THREADS;
-    if (col < d4) {
-      ((float4*)(dw + (long)v * d))[col] = acc[c];
-      q += (double)acc[c].x * acc[c].x + (double)acc[c].y * acc[c].y + (double)acc[c].z * acc[c].z +
-           (double)acc[c].w * acc[c].w;
-    }
-  }
+  if (aok) dw[(long)v * d + col0 + t] = acc;
   if (sq) {
     __shared__ double qred[EMB_THREADS / 64];
-    q = block_sum<double, EMB_THREADS>(q, qred);
-    if (t == 0) sq[blockIdx.x] = q;
+    const double q = block_sum<double, EMB_THREADS>(aok ? (double)acc * acc : 0.0, qred);
+    if (t == 0) sq[blockIdx.x + gridDim.x * blockIdx.y] = q;
   }
 }
 
@@ -517,8 +539,9 @@ extern "C" int sj_embedding_bwd(void* stream, const float* dy, const int32_t* id
   SJ_REQUIRE(n >= 0 && d > 0 && d <= 8 * EMB_THREADS && vocab > 0, "embedding_backward: n %ld d %ld vocab %ld", n,
              d, vocab);
   if (d % 4 == 0 && d <= 8 * EMB_THREADS && ((uintptr_t)dy & 15) == 0 && ((uintptr_t)dw & 15) == 0) {
-    hipLaunchKernelGGL(k_embedding_bwd4, dim3((unsigned)vocab), dim3(EMB_THREADS), 0, (hipStream_t)stream, dy, ids, dw,
-                       n, d, sjh::grad_sq().take(vocab));
+    const long chunks = (d + EMB_COLS - 1) / EMB_COLS;
+    hipLaunchKernelGGL(k_embedding_bwd4, dim3((unsigned)vocab, (unsigned)chunks), dim3(EMB_THREADS), 0,
+                       (hipStream_t)stream, dy, ids, dw, n, d, sjh::grad_sq().take(vocab * chunks));
   } else {
     hipLaunchKernelGGL(k_embedding_bwd, dim3((unsigned)vocab), dim3(EMB_THREADS), 0, (hipStream_t)stream, dy, ids, dw,
                        n, d);

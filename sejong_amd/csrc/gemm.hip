@@ -12,7 +12,10 @@
 // fp32 operands are written to LDS as two bf16 planes (hi = RNE(x),
 // lo = RNE(x - hi)) and multiplied as hi*hi + hi*lo + lo*hi, which keeps
 // fp32 gradients (the reference's fp32 "ieee" dot, kernels.py:29) to ~2^-16
-// relative on bf16 MFMA.  Global tiles are register double-buffered.
+// relative on bf16 MFMA.  Global tiles are fetched into registers several
+// k-steps ahead (PD): these calls are small (one to a few workgroups per CU,
+// K of 4 to 12 steps), and with one step in flight each step waited for its
+// own load.
 //
 // Epilogues fuse the op that follows each projection in Block::apply
 // (crates/sejong-model/src/architecture.rs:200-247): QKV + RoPE, gate/up +
@@ -30,6 +33,11 @@ namespace {
 constexpr int NT = 256;
 constexpr int BK = 32;
 constexpr int LDSK = BK + 8;  // padded row (bf16 elements)
+
+// fp32 vectors at any 4-byte address (a row stride of 257 floats is common
+// here: the vocabulary); the hardware takes them
+typedef float f4a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2a4 __attribute__((ext_vector_type(2), aligned(4)));
 
 enum Epi { EPI_STORE = 0, EPI_QKV = 1, EPI_RESID = 2, EPI_GATEUP = 3, EPI_SWIGLU_BWD = 4, EPI_PARTIAL = 5 };
 
@@ -109,7 +117,7 @@ struct Loader {
         } else {
           const float* src = (const float*)base + row * ld + k;
           if (full) {
-            float4 v0 = *(const float4*)src, v1 = *(const float4*)(src + 4);
+            const f4a4 v0 = *(const f4a4*)src, v1 = *(const f4a4*)(src + 4);
             reg[p][0] = __float_as_uint(v0.x); reg[p][1] = __float_as_uint(v0.y);
             reg[p][2] = __float_as_uint(v0.z); reg[p][3] = __float_as_uint(v0.w);
             reg[p][4] = __float_as_uint(v1.x); reg[p][5] = __float_as_uint(v1.y);
@@ -143,7 +151,7 @@ struct Loader {
           if (full) {
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-              float2 v = *(const float2*)(src + (long)i * ld);
+              const f2a4 v = *(const f2a4*)(src + (long)i * ld);
               reg[p][2 * i] = __float_as_uint(v.x);
               reg[p][2 * i + 1] = __float_as_uint(v.y);
             }
@@ -255,9 +263,11 @@ __global__ __launch_bounds__(NT) void k_gemm(GemmParams p) {
     kend = kbeg + p.kchunk < p.K ? kbeg + p.kchunk : p.K;
   }
 
-  Loader<AK, BM> la;
-  Loader<BKND, BN> lb0;
-  Loader<BKND, BN> lb1;
+  // k-steps in flight: as many as the registers of a tile leave room for
+  constexpr int PD = BM * BN > 64 * 64 ? 2 : DUAL ? 3 : 4;
+  Loader<AK, BM> la[PD];
+  Loader<BKND, BN> lb0[PD];
+  Loader<BKND, BN> lb1[DUAL ? PD : 1];
 
   f32x4 acc[NB_MAT][MB][NB];
 #pragma unroll
@@ -267,29 +277,34 @@ __global__ __launch_bounds__(NT) void k_gemm(GemmParams p) {
 #pragma unroll
       for (int j = 0; j < NB; j++) acc[q][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  auto fetch = [&](long k0) {
-    la.fetch(p.a, p.lda, m0, p.M, k0, kend, p.a_vec);
-    lb0.fetch(bptr0, ldb0, nl0, nseg_cols, k0, kend, p.b_vec);
-    if constexpr (DUAL) lb1.fetch(p.b[1], p.ldb[1], nl0, nseg_cols, k0, kend, p.b_vec);
+  auto fetch = [&](int u, long k0) {
+    la[u].fetch(p.a, p.lda, m0, p.M, k0, kend, p.a_vec);
+    lb0[u].fetch(bptr0, ldb0, nl0, nseg_cols, k0, kend, p.b_vec);
+    if constexpr (DUAL) lb1[u].fetch(p.b[1], p.ldb[1], nl0, nseg_cols, k0, kend, p.b_vec);
   };
   auto stage_ptr = [&](int s) { return lds + s * STAGE; };
-  auto store = [&](int s) {
+  auto store = [&](int u, int s) {
     bf16_t* base = stage_ptr(s);
-    la.store(base, AF ? base + ASZ : nullptr);
+    la[u].store(base, AF ? base + ASZ : nullptr);
     bf16_t* bb = base + APL * ASZ;
-    lb0.store(bb, BF ? bb + BSZ : nullptr);
-    if constexpr (DUAL) lb1.store(bb + BPL * BSZ, BF ? bb + BPL * BSZ + BSZ : nullptr);
+    lb0[u].store(bb, BF ? bb + BSZ : nullptr);
+    if constexpr (DUAL) lb1[u].store(bb + BPL * BSZ, BF ? bb + BPL * BSZ + BSZ : nullptr);
   };
 
   const int fr = lane & 15, fk = (lane >> 4) * 8;
-  if (kbeg < kend) {
-    fetch(kbeg);
-    store(0);
-    __syncthreads();
-    int cur = 0;
-    for (long k0 = kbeg; k0 < kend; k0 += BK) {
-      const bool more = k0 + BK < kend;
-      if (more) fetch(k0 + BK);
+  const int steps = (int)((kend - kbeg + BK - 1) / BK);
+#pragma unroll
+  for (int u = 0; u < PD; u++)
+    if (u < steps) fetch(u, kbeg + (long)u * BK);
+  for (int it0 = 0; it0 < steps; it0 += PD) {
+#pragma unroll
+    for (int u = 0; u < PD; u++) {
+      const int it = it0 + u, cur = it & 1;
+      if (it >= steps) continue;
+      // buffer `cur` was last read in step it - 2, before step it - 1's barrier
+      store(u, cur);
+      __syncthreads();
+      if (it + PD < steps) fetch(u, kbeg + (long)(it + PD) * BK);
       const bf16_t* base = stage_ptr(cur);
       bf16x8 ah[MB], al[MB];
 #pragma unroll
@@ -314,11 +329,6 @@ __global__ __launch_bounds__(NT) void k_gemm(GemmParams p) {
             if constexpr (AF) acc[q][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh, acc[q][i][j], 0, 0, 0);
           }
         }
-      }
-      if (more) {
-        store(cur ^ 1);
-        __syncthreads();
-        cur ^= 1;
       }
     }
   }
@@ -450,7 +460,7 @@ inline int kind_of(int dtype, bool kcontig) { return (dtype == SJ_F32 ? 2 : 0) +
 inline bool aligned(const void* ptr, long ld, int dtype, bool kcontig) {
   uintptr_t a = (uintptr_t)ptr;
   if (dtype == SJ_BF16) return kcontig ? (a % 16 == 0 && ld % 8 == 0) : (a % 4 == 0 && ld % 2 == 0);
-  return kcontig ? (a % 16 == 0 && ld % 4 == 0) : (a % 8 == 0 && ld % 2 == 0);
+  return a % 4 == 0;
 }
 
 int g_num_cu = 0;

@@ -97,6 +97,8 @@ struct FParams {
   double* sq;
   // tile order: row panels per group (0: the smaller tile dimension fastest)
   int group;
+  // k_gemm_pp: tiles in n, in m, and K slices (its grid is one-dimensional)
+  unsigned ptx, pty, ptz;
 };
 
 // Grouped tile order (row panels per group) when the B panels of one row of
@@ -1072,6 +1074,354 @@ __global__ __launch_bounds__(NT) void k_gemm_kw(FParams p) {
   }
 }
 
+// ------------------------------------------------ large products (ping-pong)
+// The same products as k_gemm_fast for shapes whose large tiles fill the
+// chip.  There one 64 x 64 (or 32 x 64, two planes) block per wave, a stage of
+// 64 k and a barrier per stage left the matrix cores at 27-40%: a wave reads
+// its fragments, waits, multiplies, and the waves of a workgroup do each at
+// the same time.  Here a workgroup is eight waves, two per SIMD, over a tile
+// whose stage of 32 k is always 512 operand rows (32 KB): 256 x 256 (one
+// plane each), 128 x 256 (two planes of A), 256 x 128 (two planes of Y, or
+// gate and up).  Per stage a wave reads 12 fragments for 32 MFMAs (k_gemm_fast
+// reads 16).  The two waves of a SIMD alternate: waves 0-3 read their
+// fragments (and issue their share of the DMA) while waves 4-7 multiply, a
+// barrier, then the other way round, so each SIMD always has a wave in its
+// 512 MFMA cycles.  Four stages of LDS form a ring: a stage's buffer is free
+// once both groups have read it, its DMA is issued three stages ahead, and
+// the wait before a barrier covers the stage the other side reads next.
+//
+// MFMA operands are passed B first, so a lane's four results are four
+// neighbouring columns of one row; two column blocks trade halves between
+// neighbouring 16-lane rows (v_permlane16_swap) and a lane holds eight, so
+// every epilogue works on registers with 16-byte accesses and no LDS.  A
+// workgroup therefore walks its tiles (one resident per CU) and starts the
+// next tile's first three stages before it stores the current one: with a
+// workgroup per tile the fill and the stores of 16384 x 2752 x 1024 took as
+// long as its products.  The sums run over k in the same order (per 32 k: hi,
+// then the other plane), so results equal k_gemm_fast's bit for bit (Delta
+// sums its head's columns in another order).  At 16384 x 1024 x 5504, two
+// planes: 420 -> 309 us, 1.2 PFLOP/s, matrix cores 61% busy (27-40% before).
+constexpr int PP_T = 512, PP_K = 32, PP_STAGE = 512 * PP_K;  // threads, k per stage, elements per stage
+constexpr size_t PP_LDS = (size_t)4 * PP_STAGE * 2;
+
+template <int PA, int PB, int EPI>
+struct PPShape {
+  static constexpr bool DUAL = EPI == E_GATEUP;
+  static constexpr int BM = PA == 2 ? 128 : 256, BN = PB == 2 || DUAL ? 128 : 256;
+};
+
+template <int PA, int PB, int EPI, int TM>
+__global__ __launch_bounds__(PP_T, 2) void k_gemm_pp(FParams p) {
+  constexpr bool TN = TM == 3, DUAL = EPI == E_GATEUP;
+  constexpr int BM = PPShape<PA, PB, EPI>::BM, BN = PPShape<PA, PB, EPI>::BN, NBM = DUAL ? 2 : 1;
+  static_assert(BM * PA + BN * PB * NBM == 512, "a stage is 512 operand rows");
+  static_assert(!(PA == 2 && PB == 2), "one split operand");
+  static_assert(EPI == E_STORE || EPI == E_PARTIAL || EPI == E_RESID || EPI == E_GATEUP || EPI == E_PLANES, "epilogue");
+  constexpr int WM = BM / 2, WN = BN / 4, MB = WM / 16, NB = WN / 16;
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];  // 4 stages
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave & 1, wn = wave >> 1;  // both groups of a SIMD pair share no accumulators
+  const unsigned nx = p.ptx, ny = p.pty, nb = nx * ny * p.ptz;
+  auto fdiv = [](unsigned n, unsigned long long mg) { return (unsigned)(((unsigned long long)n * mg) >> 40); };
+  long m0 = 0, n0 = 0;
+  unsigned tz = 0;
+  // tile v of the walk (tile order as in k_gemm_fast: a contiguous run per XCD)
+  auto locate = [&](unsigned v) {
+    unsigned logical = v;
+    if (p.xcd_remap) {
+      const unsigned xcd = v & 7, local = v >> 3, q8 = nb >> 3, r8x = nb & 7;
+      logical = xcd * q8 + (xcd < r8x ? xcd : r8x) + local;
+    }
+    tz = fdiv(logical, p.mdiv_xy);
+    const unsigned in = logical - tz * nx * ny;
+    unsigned tx, ty;
+    if (p.group > 0) {
+      const unsigned pgrp = (unsigned)p.group, ning = pgrp * nx, gid = in / ning, first = gid * pgrp;
+      const unsigned gs = ny - first < pgrp ? ny - first : pgrp, loc = in - gid * ning;
+      ty = first + loc % gs;
+      tx = loc / gs;
+    } else if (ny < nx) {
+      tx = fdiv(in, p.mdiv_lo);
+      ty = in - tx * ny;
+    } else {
+      ty = fdiv(in, p.mdiv_lo);
+      tx = in - ty * nx;
+    }
+    m0 = (long)ty * BM;
+    n0 = (long)tx * BN;
+  };
+
+  // ---- DMA: wave w stages operand rows 64 w .. + 63 of every stage (one
+  // plane of one operand), four 1 KB blocks.  k-contiguous: a block is 16
+  // rows of 64 bytes, chunk c of row r at slot c ^ ((r >> 1) & 3) (eight
+  // consecutive rows' chunk c on distinct banks).  Row
+  // layout: sub-tile w (64 columns), a block is 8 k-rows of 128 bytes, chunk
+  // c of k-row r at slot c ^ swt(r).  Rows and columns past the operand
+  // repeat its last ones (their results are not stored); k past the range
+  // (the last stage of a ragged K) reads `zero`.
+  const bf16_t* zero = (const bf16_t*)g_zero16;
+  asm volatile("" : "+s"(zero));
+  const int row64 = 64 * wave;  // first operand row of this wave's share
+  uint32_t voff[4];
+  const uint8_t* src = nullptr;
+  long kstr = 0, klen = 0;  // bytes per stage, k range
+  int nk = 0;
+  auto setup = [&]() {
+    long kbeg = 0, kend = p.K;
+    if constexpr (EPI == E_PARTIAL) {
+      kbeg = (long)tz * p.kchunk;
+      kend = kbeg + p.kchunk < p.K ? kbeg + p.kchunk : p.K;
+    }
+    klen = kend - kbeg;
+    nk = (int)((klen + PP_K - 1) / PP_K);
+    const bf16_t* base;
+    long ld, first, count;
+    if (row64 < BM * PA) {
+      const int pl = row64 / BM;
+      base = PA == 2 && pl ? p.a[1] : p.a[0];
+      ld = p.lda;
+      first = m0 + row64 % BM;
+      count = p.M;
+    } else {
+      const int rb = row64 - BM * PA, q = rb / (BN * PB), pl = (rb % (BN * PB)) / BN;
+      first = n0 + rb % BN;
+      count = p.N;
+      base = DUAL ? p.b[0][q] : pl ? p.b[1][0] : p.b[0][0];
+      ld = DUAL ? p.ldb[q] : p.ldb[0];
+    }
+    if (first >= count) first = count - (TN ? 8 : 1);  // a wholly masked share
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      if constexpr (TN) {
+        const int kr = 8 * j + (lane >> 3);
+        long col = first + 8 * ((lane & 7) ^ swt(kr));
+        col = col < count ? col : count - 8;
+        voff[j] = (uint32_t)((kr * ld + (col - first)) * 2);
+      } else {
+        long row = first + 16 * j + (lane >> 2);
+        row = row < count ? row : count - 1;
+        voff[j] = (uint32_t)(((row - first) * ld + ((lane & 3) ^ ((lane >> 3) & 3)) * 8) * 2);
+      }
+    }
+    src = uniform_ptr(TN ? base + kbeg * ld + first : base + first * ld + kbeg);
+    kstr = TN ? (long)PP_K * ld * 2 : (long)PP_K * 2;
+  };
+  const uint32_t lds_wave =
+      __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void*)lds) + (uint32_t)(wave * 64 * PP_K * 2);
+  auto issue = [&](int it) {
+    const uint32_t sb = lds_wave + (uint32_t)((it & 3) * PP_STAGE * 2);
+    const uint8_t* bs = src + it * kstr;
+    if ((long)(it + 1) * PP_K <= klen) {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:0" ::"v"(voff[j]), "s"(bs),
+                     "s"(sb + (uint32_t)(j * 1024))
+                     : "memory", "m0");
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        // the lane's last k of the block
+        const int kp = TN ? 8 * j + (lane >> 3) : ((lane & 3) ^ ((lane >> 3) & 3)) * 8 + 7;
+        dma16((long)it * PP_K + kp < klen ? (const void*)(bs + voff[j]) : (const void*)zero, sb + (uint32_t)(j * 1024));
+      }
+    }
+  };
+  auto fill = [&]() {
+#pragma unroll
+    for (int it = 0; it < 3; it++)
+      if (it < nk) issue(it);
+  };
+
+  // ---- fragments of one stage: A blocks i (planes), B blocks j (planes or halves)
+  const int fr = lane & 15, fg = lane >> 4;
+  const int lo = fr * PP_K + ((fg ^ ((fr >> 1) & 3)) << 3);  // this lane's chunk of a 16-row block
+  constexpr int NFB = NB * PB * NBM;
+  bf16x8 fa[PA][MB], fb[NFB];
+  auto read = [&](int it) {
+    const bf16_t* st = lds + (it & 3) * PP_STAGE;
+#pragma unroll
+    for (int q = 0; q < PB * NBM; q++)
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        const int r = BM * PA + q * BN + wn * WN + 16 * j;  // operand row of the block
+        if constexpr (TN)
+          fb[q * NB + j] = tr_frag(st + (r / 64) * 64 * PP_K, 0, r % 64, lane);
+        else
+          fb[q * NB + j] = __builtin_bit_cast(bf16x8, *(const u32x4*)(st + r * PP_K + lo));
+      }
+#pragma unroll
+    for (int pl = 0; pl < PA; pl++)
+#pragma unroll
+      for (int i = 0; i < MB; i++) {
+        const int r = pl * BM + wm * WM + 16 * i;
+        if constexpr (TN)
+          fa[pl][i] = tr_frag(st + (r / 64) * 64 * PP_K, 0, r % 64, lane);
+        else
+          fa[pl][i] = __builtin_bit_cast(bf16x8, *(const u32x4*)(st + r * PP_K + lo));
+      }
+  };
+  f32x4 acc[NBM][MB][NB];
+  auto multiply = [&]() {
+#pragma unroll
+    for (int pl = 0; pl < (PA == 2 || PB == 2 ? 2 : 1); pl++)
+#pragma unroll
+      for (int q = 0; q < NBM; q++)
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+          for (int i = 0; i < MB; i++)
+            acc[q][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[(DUAL ? q : PB == 2 ? pl : 0) * NB + j],
+                                                                   fa[PA == 2 ? pl : 0][i], acc[q][i][j], 0, 0, 0);
+  };
+
+  unsigned v = blockIdx.x;  // gridDim.x <= nb
+  locate(v);
+  setup();
+  fill();
+  for (;;) {
+#pragma unroll
+    for (int q = 0; q < NBM; q++)
+#pragma unroll
+      for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) acc[q][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // ---- ring of four stages, groups half a step apart.  The waits count
+    // the DMA of later stages; stores still in flight from the tile before
+    // only make them stricter.
+    wait_stages<4, 2>(nk - 1 < 2 ? nk - 1 : 2);  // stage 0 has landed
+    asm volatile("s_barrier" ::: "memory");
+    if (wave >= 4) asm volatile("s_barrier" ::: "memory");
+    for (int it = 0; it < nk; it++) {
+      read(it);
+      // buffer (it + 3) & 3 held stage it - 1: both groups' reads of it ended
+      // before the barrier that opened this half step
+      if (it + 3 < nk) issue(it + 3);
+      __builtin_amdgcn_sched_barrier(0);
+      const int after = nk - 2 - it < 2 ? nk - 2 - it : 2;  // stages after it + 1 in flight
+      wait_stages<4, 2>(after > 0 ? after : 0);             // stage it + 1 has landed
+      block_barrier();                                      // (and this stage's reads)
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+      multiply();
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_barrier" ::: "memory");
+    }
+    if (wave < 4) asm volatile("s_barrier" ::: "memory");
+    // every read of the ring is done (both groups are past their last)
+
+    // ---- epilogue: acc[q][i][j][r] = C[m0 + wm WM + 16 i + fr][n0 + wn WN + 16 j + 4 fg + r]
+    const long mt = m0 + wm * WM + fr, nt = n0 + wn * WN;
+    const unsigned tzc = tz;
+    // after the exchange of column blocks j, j + 1: this lane's 8 columns
+    const int n8 = 16 * (fg & 1) + 8 * (fg >> 1);
+    constexpr bool F32 = EPI == E_STORE || EPI == E_PARTIAL;
+    u32x4 res[EPI == E_RESID ? MB : 1][NB / 2];
+    if constexpr (EPI == E_RESID) {  // the residual: all requested before the next tile's DMA
+#pragma unroll
+      for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j += 2) {
+          const long m = mt + 16 * i, n = nt + 16 * j + n8;
+          res[i][j / 2] = m < p.M && n < p.N ? *(const u32x4*)(p.r + m * p.ldr + n) : u32x4{0u, 0u, 0u, 0u};
+        }
+    }
+    const unsigned vn = v + gridDim.x;
+    if (vn < nb) {  // uniform
+      locate(vn);
+      setup();
+      fill();
+    }
+#pragma unroll
+    for (int i = 0; i < MB; i++) {
+      const long m = mt + 16 * i;
+      float dpart = 0.f;
+#pragma unroll
+      for (int j = 0; j < NB; j += 2) {
+        if constexpr (F32) {
+#pragma unroll
+          for (int jj = j; jj < j + 2; jj++) {
+            const long n = nt + 16 * jj + 4 * fg;
+            if (m >= p.M || n >= p.N) continue;  // N % 8 == 0: a lane's columns are in or out together
+            const f32x4 x = acc[0][i][jj];
+            if (EPI == E_STORE && p.c_bf16) {
+              *(u32x2*)((bf16_t*)p.c[0] + m * p.ldc[0] + n) =
+                  u32x2{pack2(f2bf(x[0]), f2bf(x[1])), pack2(f2bf(x[2]), f2bf(x[3]))};
+            } else {
+              float* d = EPI == E_PARTIAL ? p.partial + ((long)tzc * p.M + m) * p.N + n
+                                          : (float*)p.c[0] + m * p.ldc[0] + n;
+              float4 o = make_float4(x[0], x[1], x[2], x[3]);
+              if (EPI == E_STORE && p.accumulate) {
+                const float4 c = *(const float4*)d;
+                o = make_float4(c.x + o.x, c.y + o.y, c.z + o.z, c.w + o.w);
+              }
+              *(float4*)d = o;
+            }
+          }
+        } else {
+          const long n = nt + 16 * j + n8;
+          const bool ok = m < p.M && n < p.N;
+          float x[NBM][8];
+#pragma unroll
+          for (int q = 0; q < NBM; q++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[q][i][j][r]),
+                                                              __float_as_uint(acc[q][i][j + 1][r]), false, false);
+              x[q][r] = __uint_as_float(w[0]);
+              x[q][4 + r] = __uint_as_float(w[1]);
+            }
+          if (!ok) continue;
+          auto put8 = [&](bf16_t* d, const bf16_t* e) {
+            *(u32x4*)d = u32x4{pack2(e[0], e[1]), pack2(e[2], e[3]), pack2(e[4], e[5]), pack2(e[6], e[7])};
+          };
+          bf16_t e0[8], e1[8], e2[8];
+          if constexpr (EPI == E_RESID) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) e0[r] = f2bf(bf_word(res[i][j / 2], r) + round_bf(x[0][r]));
+            put8((bf16_t*)p.c[0] + m * p.ldc[0] + n, e0);
+          } else if constexpr (EPI == E_GATEUP) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+              const float gv = round_bf(x[0][r]), uv = round_bf(x[NBM - 1][r]);
+              e0[r] = f2bf(gv);
+              e1[r] = f2bf(uv);
+              e2[r] = f2bf(gv * sigm(gv) * uv);
+            }
+            const long o = m * p.ldc[0] + n;
+            put8((bf16_t*)p.c[0] + o, e0);
+            put8((bf16_t*)p.c[1] + o, e1);
+            put8((bf16_t*)p.c[2] + o, e2);
+          } else {  // E_PLANES
+#pragma unroll
+            for (int r = 0; r < 8; r++) split_bf(x[0][r], e0[r], e1[r]);
+            put8((bf16_t*)p.c[0] + m * p.ldc[0] + n, e0);
+            put8((bf16_t*)p.c[1] + m * p.ldc[0] + n, e1);
+            if (p.delta) {
+              const u32x4 ow = *(const u32x4*)(p.o + m * p.ldo + n);
+#pragma unroll
+              for (int r = 0; r < 8; r++) dpart += (bf2f(e0[r]) + bf2f(e1[r])) * bf_word(ow, r);
+            }
+          }
+        }
+      }
+      if constexpr (EPI == E_PLANES) {
+        // the wave's 64 columns are one head: 16 of them per lane, then the four lanes of the row
+        static_assert(EPI != E_PLANES || WN == 64, "a head per wave");
+        if (p.delta) {
+          dpart += __shfl_xor(dpart, 16, 64);
+          dpart += __shfl_xor(dpart, 32, 64);
+          if (fg == 0 && m < p.M && nt < p.N) p.delta[(nt / 64) * p.lddelta + m] = dpart;
+        }
+      }
+    }
+    if (vn >= nb) break;
+    v = vn;
+  }
+}
+
 // sq (nullable): FP64 sum of squares of the values this workgroup stores,
 // at sq[blockIdx.x] (the gradient-norm hook)
 __global__ __launch_bounds__(256) void k_reduce_partials(const float* __restrict__ partial, int splits, long M, long N,
@@ -1182,6 +1532,36 @@ int launch_kw(hipStream_t s, const FParams& p, int pb, int splits) {
   return pb == 2 ? launch_kw_ns<2, EPI, 2>(s, p, splits) : launch_kw_ns<1, EPI, 2>(s, p, splits);
 }
 
+int cus();
+template <int PA, int PB, int EPI, int TM>
+int launch_pp(hipStream_t s, const FParams& p, int splits) {
+  constexpr int BM = PPShape<PA, PB, EPI>::BM, BN = PPShape<PA, PB, EPI>::BN;
+  auto kern = k_gemm_pp<PA, PB, EPI, TM>;
+  FParams& q = const_cast<FParams&>(p);
+  q.xcd_remap = xcd_remap();
+  q.ptx = (unsigned)((p.N + BN - 1) / BN);
+  q.pty = (unsigned)((p.M + BM - 1) / BM);
+  q.ptz = (unsigned)splits;
+  q.group = tile_group(p.N * (EPI == E_GATEUP ? 2 : 1), p.K, PB, q.pty);
+  const unsigned long long nb = (unsigned long long)q.ptx * q.pty * q.ptz;
+  if (nb >= (1ull << 20)) return sjh::fail(SJ_ERR_INVALID, "gemm: %u x %u x %u tiles (at most 2^20)", q.ptx, q.pty, q.ptz);
+  auto magic = [](unsigned long long d) { return (1ull << 40) / d + 1; };
+  q.mdiv_lo = magic(q.pty < q.ptx ? q.pty : q.ptx);
+  q.mdiv_xy = magic((unsigned long long)q.ptx * q.pty);
+  // one workgroup per CU walks the tiles; a multiple of 8 keeps a walk on its XCD's run
+  const unsigned slots = (unsigned)(cus() / 8 * 8);
+  const dim3 grid(nb < slots || slots == 0 ? (unsigned)nb : slots);
+  sjh::ProfHook& h = sjh::prof_hook();
+  if (h.on && h.k0) {
+    hipExtLaunchKernelGGL(kern, grid, dim3(PP_T), (uint32_t)PP_LDS, s, h.k0, h.k1, 0u, p);
+    h.used = true;
+  } else {
+    hipLaunchKernelGGL(kern, grid, dim3(PP_T), PP_LDS, s, p);
+  }
+  if (h.on) snprintf(h.kernel, sizeof(h.kernel), "k_gemm_pp<%d, %d, %d, %d>", PA, PB, EPI, TM);
+  return SJ_OK;
+}
+
 // Pipeline depth (measured on gfx950 over the cfg2 and cfg5 step GEMMs):
 // three stages when every workgroup of the launch is resident at three
 // (deeper prefetch, nothing gained by more residency); otherwise two when
@@ -1190,7 +1570,6 @@ int launch_kw(hipStream_t s, const FParams& p, int pb, int splits) {
 // occupancy query (LDS and registers of that instantiation).
 // SJ_GEMM_STAGES=2|3 overrides it (sweeps).
 int g_stages = -1;
-int cus();
 template <int BM, int BN, int PA, int PB, int EPI, int NS, int TM = 0>
 int resident() {
   static int occ = -1;
@@ -1498,6 +1877,87 @@ int launch_planes_one(hipStream_t s, const FParams& p, int pa, int pb, int bm, i
 
 bool ok16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
+constexpr int PP_SPLITS = 8;  // K slices of a dW product at most
+// The ping-pong kernel's modelled time, us: rounds of one tile per CU, each a
+// fixed part (fill, epilogue) and stages of 32 k that take a0 + a1 x the share
+// of the CUs at work (the chip's matrix rate levels off near 1 PFLOP/s).
+double pp_us(long t, double stages, double fixed, double a0, double a1) {
+  const long cu = cus();
+  const double share = t < cu ? (double)t / (double)cu : 1.0;
+  return (double)((t + cu - 1) / cu) * (fixed + stages * (a0 + a1 * share));
+}
+
+// Whether the ping-pong kernel is the faster one for the epilogue's product of
+// k-contiguous operands.  Both sides are modelled from twelve block shapes of
+// 2048-16384 rows and widths of 384-1024 (us, k_gemm_fast -> k_gemm_pp):
+//   gate|up      16384 x 2752 x 1024 278 -> 228, 8000 x 2048 x 768 97 -> 74,
+//                4096 x 1024 x 384 19 -> 24, 6000 x 1376 x 512 46 -> 48
+//   residual     16384 x 1024 x 2752 122 -> 98, 8192 x 1024 x 1024 31 -> 40
+//   dX           8000 x 768 x 4096 141 -> 110, 4096 x 1024 x 3072 58 -> 70
+//   split output 8192 x 1024 x 1024 53 -> 45, 4096 x 1024 x 1024 27 -> 34
+// Its per-tile cost is higher (one tile per CU, 128 KB of LDS), so it wins
+// where the tiles fill the chip.  The QKV (16384 x 1536 x 1024: 89 -> 95) and
+// SwiGLU-derivative (16384 x 2752 x 1024: 298 -> 308) epilogues did not win
+// at any shape and stay with k_gemm_fast.
+bool pp_wins(int epi, long M, long N, long K) {
+  const double mn = (double)M * (double)N, st = (double)K / PP_K, fl = 2.0 * mn * (double)K;
+  double pp, old;
+  if (epi == E_GATEUP) {
+    pp = pp_us(tiles(M, N, 256, 128), st, 18.0, 0.65, 0.0);
+    old = 4.0 + 2.0 * fl / 0.75e9 + 6.0 * mn / 4e6;
+  } else if (epi == E_RESID) {
+    pp = pp_us(tiles(M, N, 256, 256), st, 14.0, 0.55, 0.42);
+    old = 4.0 + fl / 0.9e9 + 4.0 * mn / 4e6;
+  } else if (epi == E_PLANES) {
+    pp = pp_us(tiles(M, N, 128, 256), st, 12.0, 0.5, 0.4);
+    old = 4.0 + 2.0 * fl / 0.78e9 + 6.0 * mn / 4e6;
+  } else {  // E_STORE, A in two planes
+    pp = pp_us(tiles(M, N, 128, 256), st, 8.0, 0.5, 0.4);
+    old = 4.0 + 2.0 * fl / 0.78e9 + 4.0 * mn / 4e6;
+  }
+  return pp < 0.9 * old;
+}
+
+// The same for a dW product (both operands in row layout, Y in two planes),
+// with its K slices.  k_gemm_fast's time follows its plan: stages of 64 k at
+// 1.42 us for a 128 x 128 tile (one per CU), 1.05 for 128 x 64 (two) and 0.78
+// for 64 x 64 (three); k_gemm_kw's steps of 128 tokens take 0.8.  (us:
+// 1024 x 5504 x 16384 715 -> 447, 1024 x 5504 x 5000 219 -> 150, 2048 x 768 x
+// 8000 100 -> 71, 1024 x 1024 x 4096 30 -> 42, 2752 x 1024 x 2048 36 -> 43.)
+bool pp_wins_dw(long M, long N, long K, int& splits) {
+  splits = 1;
+  const double mn = (double)M * (double)N;
+  const long t = tiles(M, N, 256, 128), cu = cus();
+  double best = 0;
+  for (int s = 1; s <= PP_SPLITS && (s == 1 || K / s >= 1024); s++) {
+    const double c = pp_us(t * s, (double)K / PP_K / s, 6.0, 0.45, 0.55) + (s > 1 ? 4.0 + s * mn * 8.0 / 4.5e6 : 0.0);
+    if (s == 1 || c < best) {
+      best = c;
+      splits = s;
+    }
+  }
+  int bm, bn, so;
+  double old;
+  if (plan_kw(M, N, K, 1, so)) {
+    old = 2.0 + (double)K / 128 / so * 0.8;
+  } else {
+    plan(M, N, K, 1, bm, bn, so, true);
+    const bool one = bm == 128 && bn == 128;
+    const long slots = one ? cu : bm + bn == 192 ? 2 * cu : 3 * cu;
+    old = 3.0 + (double)((tiles(M, N, bm, bn) * so + slots - 1) / slots) * ((double)K / 64 / so) *
+                    (one ? 1.42 : bm + bn == 192 ? 1.05 : 0.78);
+  }
+  if (so > 1) old += 4.0 + so * mn * 8.0 / 4.5e6;
+  return best < 0.92 * old;
+}
+// bf16 outputs (and inputs) of the ping-pong epilogues: 16-byte accesses of eight columns
+bool pp_cols_ok(const FParams& p, int nout) {
+  if (p.N % 8 || p.ldc[0] % 8) return false;
+  for (int i = 0; i < nout; i++)
+    if (!ok16(p.c[i])) return false;
+  return true;
+}
+
 // The row-plane SwiGLU epilogue moves G, U and the four planes in whole
 // 16-byte chunks: no transposed outputs, 8-aligned widths and strides.
 bool swiglu_rows_ok(const FParams& p) {
@@ -1549,6 +2009,12 @@ int set_attrs_planes() {
   return s;
 }
 
+template <int PA, int PB, int EPI, int TM>
+int set_attr_pp() {
+  hipError_t e = hipFuncSetAttribute((const void*)k_gemm_pp<PA, PB, EPI, TM>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)PP_LDS);
+  return e == hipSuccess ? SJ_OK : sjh::hip_check(e, "gemm: LDS attribute");
+}
 template <int PB, int EPI, int NS>
 int set_attr_kw() {
   hipError_t e = hipFuncSetAttribute((const void*)k_gemm_kw<PB, EPI, NS>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1585,6 +2051,12 @@ int gemm_fast_prepare() {
   if (!status) status = set_attrs_tiles<E_PARTIAL, 1, 2, 1>();
   if (!status) status = set_attrs_tiles<E_STORE, 2, 2, 2>();
   if (!status) status = set_attrs_tiles<E_PARTIAL, 2, 2, 2>();
+  if (!status) status = set_attr_pp<2, 1, E_STORE, 0>();
+  if (!status) status = set_attr_pp<1, 1, E_RESID, 0>();
+  if (!status) status = set_attr_pp<1, 1, E_GATEUP, 0>();
+  if (!status) status = set_attr_pp<2, 1, E_PLANES, 0>();
+  if (!status) status = set_attr_pp<1, 2, E_STORE, 3>();
+  if (!status) status = set_attr_pp<1, 2, E_PARTIAL, 3>();
   if (!status) status = set_attrs_tall<E_STORE>();
   if (!status) status = set_attrs_tall<E_PARTIAL>();
   if (!status) status = set_attrs_kw<E_STORE>();
@@ -1608,6 +2080,11 @@ extern "C" size_t sj_gemm_planes_workspace_bytes(long M, long N, long K) {
       const size_t b = s > 1 ? sizeof(float) * (size_t)s * (size_t)M * (size_t)N : 0;
       need = b > need ? b : need;
     }
+  int s = 1;  // the ping-pong dW plan
+  if (pp_wins_dw(M, N, K, s) && s > 1) {
+    const size_t b = sizeof(float) * (size_t)s * (size_t)M * (size_t)N;
+    need = b > need ? b : need;
+  }
   return need;
 }
 
@@ -1665,6 +2142,36 @@ int gemm_planes(void* stream, long M, long N, long K, const uint16_t* a_hi, cons
   p.c[0] = c; p.ldc[0] = ldc; p.c_bf16 = c_dtype == SJ_BF16; p.accumulate = accumulate;
   const int pa = a_lo ? 2 : 1, pb = b_lo ? 2 : 1;
   int bm, bn, splits;
+  const bool pp_out = N % 8 == 0 && ldc % 4 == 0 && ok16(c);
+  if constexpr (TM == 0) {
+    if (pp_out && pa == 2 && pb == 1 && pp_wins(E_STORE, M, N, K)) {
+      if (int st = launch_pp<2, 1, E_STORE, 0>(s, p, 1)) return st;
+      if (sjh::grad_sq().base && sjh::grad_sq().on) sjh::grad_sq().missed = true;
+      SJ_LAUNCH_CHECK("matmul planes");
+      return SJ_OK;
+    }
+  }
+  if constexpr (TM == 3) {
+    if (pp_out && pa == 1 && pb == 2 && pp_wins_dw(M, N, K, splits) &&
+        (splits == 1 || (workspace && ok16(workspace) && workspace_bytes >= sizeof(float) * (size_t)splits * M * N))) {
+      int st;
+      if (splits > 1) {
+        long kchunk = (K + splits - 1) / splits;
+        kchunk = (kchunk + PP_K - 1) / PP_K * PP_K;
+        splits = (int)((K + kchunk - 1) / kchunk);
+        p.kchunk = kchunk;
+        p.partial = (float*)workspace;
+        st = launch_pp<1, 2, E_PARTIAL, 3>(s, p, splits);
+        if (!st) st = reduce_partials(s, p, splits, workspace);
+      } else {
+        st = launch_pp<1, 2, E_STORE, 3>(s, p, 1);
+        if (sjh::grad_sq().base && sjh::grad_sq().on) sjh::grad_sq().missed = true;
+      }
+      if (st) return st;
+      SJ_LAUNCH_CHECK("matmul planes");
+      return SJ_OK;
+    }
+  }
   if constexpr (TM == 3)
     if (plan_kw(M, N, K, pa, splits)) return gemm_kw(s, p, pb, splits, workspace, workspace_bytes);
   plan(M, N, K, pa, bm, bn, splits, TM != 0);
@@ -1784,7 +2291,11 @@ extern "C" int sj_gemm_planes_split_out(void* stream, long M, long N, long K, co
   p.o = (const bf16_t*)o; p.ldo = ldo; p.delta = delta_t; p.lddelta = ld_delta;
   int bm, bn, splits;
   plan(M, N, K, 2, bm, bn, splits);
-  int st = launch_planes<E_PLANES>((hipStream_t)stream, p, 2, 1, bm, bn, 1);
+  int st;
+  if (!c_t_hi && pp_cols_ok(p, 2) && pp_wins(E_PLANES, M, N, K))
+    st = launch_pp<2, 1, E_PLANES, 0>((hipStream_t)stream, p, 1);
+  else
+    st = launch_planes<E_PLANES>((hipStream_t)stream, p, 2, 1, bm, bn, 1);
   if (st) return st;
   SJ_LAUNCH_CHECK("matmul planes out");
   return SJ_OK;
@@ -1858,7 +2369,11 @@ extern "C" int sj_gate_up_fwd_t(void* stream, const uint16_t* x, long ldx, long 
   int bm, bn;
   pick(M, F, bm, bn);
   if (bm == 128 && bn == 128) bn = 64;  // dual accumulators: keep the wave tile at 64x32
-  int st = launch_planes<E_GATEUP>((hipStream_t)stream, p, 1, 1, bm, bn, 1);
+  int st;
+  if (!h_t && pp_cols_ok(p, 3) && pp_wins(E_GATEUP, M, F, D))
+    st = launch_pp<1, 1, E_GATEUP, 0>((hipStream_t)stream, p, 1);
+  else
+    st = launch_planes<E_GATEUP>((hipStream_t)stream, p, 1, 1, bm, bn, 1);
   if (st) return st;
   SJ_LAUNCH_CHECK("gate_up");
   return SJ_OK;
@@ -1879,7 +2394,11 @@ extern "C" int sj_linear_residual_fwd_t(void* stream, const uint16_t* x, long ld
   p.M = M; p.N = N; p.K = K; p.c_bf16 = 1;
   int bm, bn;
   pick(M, N, bm, bn);
-  int st = launch_planes<E_RESID>((hipStream_t)stream, p, 1, 1, bm, bn, 1);
+  int st;
+  if (pp_cols_ok(p, 1) && ok16(r) && ldr % 8 == 0 && pp_wins(E_RESID, M, N, K))
+    st = launch_pp<1, 1, E_RESID, 0>((hipStream_t)stream, p, 1);
+  else
+    st = launch_planes<E_RESID>((hipStream_t)stream, p, 1, 1, bm, bn, 1);
   if (st) return st;
   SJ_LAUNCH_CHECK("linear_residual");
   return SJ_OK;

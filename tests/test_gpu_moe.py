@@ -276,6 +276,33 @@ def test_route_pack_all_expert_counts(api, lib, E, K):
     np.testing.assert_array_equal(pslot[PP.host()], np.arange(S))
 
 
+@pytest.mark.parametrize("S", [1, 255, 256, 257, 4097, 65536, 65537])
+@pytest.mark.parametrize("E", [1, 4, 5, 8, 9, 16])
+def test_route_pack_sizes(api, lib, S, E):
+    """The pack over many workgroups at its chunk's and its range's edges
+    (one slot past 65536: the single-workgroup form), with ids out of range
+    and, at S = 65536, every id on one expert; whole numbers, exact."""
+    rng = np.random.default_rng(S + E)
+    ids = np.full(S, E - 1) if S == 65536 else rng.integers(-1, E + 1, S)
+    ids = ids.astype(np.int32)
+    cap = lib.sj_route_pack_capacity(S, E) + 192
+    IDS, TOK, SLT = dev(ids, "i32"), zeros(E * S, "i32"), zeros(E * S, "i32")
+    CNT, OFF, PS, PP = empty(E, "i32"), empty(E + 1, "i32"), empty(cap, "i32"), empty(S, "i32")
+    api.sj_route_pack(None, IDS.p, S, 1, E, TOK.p, SLT.p, CNT.p, OFF.p, PS.p, PP.p, cap)
+    sync()
+    per = [np.flatnonzero(ids == e) for e in range(E)]
+    off = np.concatenate([[0], np.cumsum([(len(q) + 63) // 64 * 64 for q in per])])
+    pslot, ppos = np.full(cap, -1), np.full(S, -1)
+    tok = np.zeros((E, S))
+    for e, q in enumerate(per):
+        pslot[off[e]:off[e] + len(q)] = q
+        ppos[q] = off[e] + np.arange(len(q))
+        tok[e, :len(q)] = q
+    for got, ref in ((CNT, [len(q) for q in per]), (OFF, off), (PS, pslot), (PP, ppos), (TOK, tok.ravel()),
+                     (SLT, tok.ravel())):
+        np.testing.assert_array_equal(got.host(), ref)
+
+
 def test_gather_bwd_vector_form_is_bit_exact(api, lib):
     """The 16-byte gather/route backward equals the per-column kernel bit
     for bit (same per-column order); an odd dz stride selects the latter."""

@@ -219,10 +219,23 @@ __global__ __launch_bounds__(256) void k_cross_entropy_planes(const float* x, lo
 }
 
 // kernels.py:254-262 (single workgroup, FP64, fixed order)
+// A thread's loads go out 16 at a time (past the end: the last value, added as
+// zero): one after the other, 4096 tokens' rows took 16 memory latencies (5.2 ->
+// 3.5 us).
 __global__ __launch_bounds__(256) void k_loss_summary(const float* loss, long n, double* out, long slot, float weight) {
   __shared__ double red[4];
   double s = 0.0;
-  for (long i = threadIdx.x; i < n; i += 256) s += (double)loss[i];
+  constexpr int U = 16;
+  for (long i0 = threadIdx.x; i0 < n; i0 += 256 * U) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const long i = i0 + 256 * u;
+      v[u] = loss[i < n ? i : n - 1];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) s += i0 + 256 * u < n ? (double)v[u] : 0.0;
+  }
   s = block_sum<double, 256>(s, red);
   if (threadIdx.x == 0) out[slot] = s * (double)weight / (double)n;
 }

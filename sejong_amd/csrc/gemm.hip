@@ -404,8 +404,23 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const float* __restrict__
                                                        void* c, long ldc, int c_bf16, int accumulate) {
   const long total = M * N;
   for (long i = blockIdx.x * 256L + threadIdx.x; i < total; i += (long)gridDim.x * 256L) {
+    // slices in order, eight loads in flight (one at a time each slice was a
+    // memory latency: 384 x 257 of 4096 tokens 6.1 -> 4.6 us)
     float s = 0.f;
-    for (int z = 0; z < splits; z++) s += partial[(long)z * total + i];
+    int z = 0;
+    for (; z + 8 <= splits; z += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = partial[(long)(z + u) * total + i];
+#pragma unroll
+      for (int u = 0; u < 8; u++) s += v[u];
+    }
+    for (; z + 2 <= splits; z += 2) {
+      const float a = partial[(long)z * total + i], b = partial[(long)(z + 1) * total + i];
+      s += a;
+      s += b;
+    }
+    if (z < splits) s += partial[(long)z * total + i];
     const long m = i / N, n = i - m * N;
     const long idx = m * ldc + n;
     if (c_bf16)

@@ -501,7 +501,15 @@ __device__ __forceinline__ bool al16(const void* p) { return ((uintptr_t)p & 15)
 // parameter_gradient_update / _materialize / _norm (parameter.py:244-291):
 // one workgroup per 16x1024 tile of one parameter (owner from the table).
 // Action 0 materialize (G into w), 1 update, 2 FP64 sum of G^2 per tile.
-__global__ __launch_bounds__(256) void k_factored_apply(const uint8_t* __restrict__ meta, int action, float lr,
+// FU: loads of `right`, tail rows and weights in flight.  FBM (small tables,
+// bound by latency): the weights are requested first and travel under the
+// gradient's work, 211 VGPRs.  2 (tables past FSMALL tiles, bound by
+// HBM with other workgroups to switch to): the registers stay at four
+// workgroups a CU or more.  MINW keeps the compiler to that.  384 tiles (1024 x 5504):
+// 29 -> 23 us; all of 133 M parameters: norm 186 -> 154 us, update 318 -> 279
+// (the small form there 309 and 356).
+template <int FU, int MINW>
+__global__ __launch_bounds__(256, MINW) void k_factored_apply(const uint8_t* __restrict__ meta, int action, float lr,
                                                         float decay, double* __restrict__ partials,
                                                         const sj_sgd_step* __restrict__ step,
                                                         const double* __restrict__ sumsq) {
@@ -517,14 +525,17 @@ __global__ __launch_bounds__(256) void k_factored_apply(const uint8_t* __restric
   const long m0 = (local / P.col_tiles) * FBM, n = (local % P.col_tiles) * FBN + 4 * threadIdx.x;
   const int cnt = n < P.cols ? (P.cols - n < 4 ? (int)(P.cols - n) : 4) : 0;
   const bool wvec = (P.cols & 3) == 0 && (P.ld & 3) == 0 && al16(P.w) && (!P.dense || al16(P.dense));
-  float4 g[FBM], w4[FBM];
+  constexpr bool FIRST = FU == FBM;
+  constexpr int RU = FU < 8 ? FU : 8;  // rows of `right` and of a tail
+  float4 g[FBM], w4[FU];
 #pragma unroll
-  for (int i = 0; i < FBM; i++) g[i] = w4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (action == 1 && cnt > 0) {  // the weights travel under the gradient's work
+  for (int i = 0; i < FBM; i++) g[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto weights = [&](int i0) {
 #pragma unroll
-    for (int i = 0; i < FBM; i++)
-      if (m0 + i < P.rows) w4[i] = ld4(P.w + (m0 + i) * P.ld + n, cnt, wvec);
-  }
+    for (int u = 0; u < FU; u++)
+      w4[u] = m0 + i0 + u < P.rows ? ld4(P.w + (m0 + i0 + u) * P.ld + n, cnt, wvec) : make_float4(0.f, 0.f, 0.f, 0.f);
+  };
+  if (FIRST && action == 1 && cnt > 0) weights(0);
   // head = sum over the terms' ranks of (left * scale) right
   for (int ti = 0; ti < P.term_count; ti++) {
     const FTerm tm = terms[P.term_begin + ti];
@@ -540,13 +551,13 @@ __global__ __launch_bounds__(256) void k_factored_apply(const uint8_t* __restric
       if (cnt > 0) {
         // eight rows of `right` in flight (one at a time, each waited for its
         // own latency; with the tail rows below 29 -> 23 us at 1024 x 5504, rank 16)
-        for (long rb = 0; rb < rn; rb += 8) {
-          float4 rv[8];
+        for (long rb = 0; rb < rn; rb += RU) {
+          float4 rv[RU];
 #pragma unroll
-          for (int u = 0; u < 8; u++)
+          for (int u = 0; u < RU; u++)
             rv[u] = rb + u < rn ? ld4(tm.right + (r0 + rb + u) * tm.ld + n, cnt, tvec) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-          for (int u = 0; u < 8; u++) {
+          for (int u = 0; u < RU; u++) {
             if (rb + u >= rn) break;
 #pragma unroll
             for (int i = 0; i < FBM; i++) {
@@ -579,15 +590,15 @@ __global__ __launch_bounds__(256) void k_factored_apply(const uint8_t* __restric
     __syncthreads();
     if (cnt == 0) continue;
 #pragma unroll
-    for (int i0 = 0; i0 < FBM; i0 += 8) {
-      float4 tv[8];
+    for (int i0 = 0; i0 < FBM; i0 += RU) {
+      float4 tv[RU];
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
+      for (int i = 0; i < RU; i++) {
         const int sel = __builtin_amdgcn_readfirstlane(ssel[i0 + i]);
         if (sel >= 0) tv[i] = ld4(tm.tail + (long)sel * tm.ld + n, cnt, tvec);
       }
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
+      for (int i = 0; i < RU; i++) {
         const int sel = __builtin_amdgcn_readfirstlane(ssel[i0 + i]);
         if (sel >= 0) {
           float4& q = g[i0 + i];
@@ -633,13 +644,15 @@ __global__ __launch_bounds__(256) void k_factored_apply(const uint8_t* __restric
   const float keep = (P.decay && action == 1) ? 1.f - decay : 1.f;
 #pragma unroll
   for (int i = 0; i < FBM; i++) {
+    if (!FIRST && action == 1 && i % FU == 0) weights(i);
     const long m = m0 + i;
     if (m >= P.rows) continue;
     float* wp = P.w + m * P.ld + n;
     float4 o = g[i];
     if (action == 1) {
-      o = make_float4(w4[i].x * keep - lr * g[i].x, w4[i].y * keep - lr * g[i].y, w4[i].z * keep - lr * g[i].z,
-                      w4[i].w * keep - lr * g[i].w);
+      const float4 wi = w4[i % FU];
+      o = make_float4(wi.x * keep - lr * g[i].x, wi.y * keep - lr * g[i].y, wi.z * keep - lr * g[i].z,
+                      wi.w * keep - lr * g[i].w);
     }
     if (wvec && cnt == 4) {
       *(float4*)wp = o;
@@ -942,13 +955,24 @@ extern "C" int sj_factored_pack(const sj_factored_param* params, long nparams, c
   return SJ_OK;
 }
 
+namespace {
+constexpr long FSMALL = 1024;  // two rounds of the small form's two workgroups on 256 CUs
+void launch_factored(hipStream_t s, const void* meta, long tiles, int action, float lr, float decay, double* partials,
+                     const sj_sgd_step* step, const double* sumsq) {
+  if (tiles <= FSMALL)
+    hipLaunchKernelGGL((k_factored_apply<FBM, 2>), dim3((unsigned)tiles), dim3(256), 0, s, (const uint8_t*)meta, action,
+                       lr, decay, partials, step, sumsq);
+  else
+    hipLaunchKernelGGL((k_factored_apply<2, 4>), dim3((unsigned)tiles), dim3(256), 0, s, (const uint8_t*)meta, action,
+                       lr, decay, partials, step, sumsq);
+}
+}  // namespace
+
 extern "C" int sj_factored_apply(void* stream, const void* meta, long tiles, int action, float lr, float decay,
                                  double* partials) {
   SJ_REQUIRE(meta && tiles > 0 && tiles < (1L << 31) && action >= 0 && action <= 2 && (action != 2 || partials),
              "compact SGD apply: action %d", action);
-  hipLaunchKernelGGL(k_factored_apply, dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream,
-                     (const uint8_t*)meta, action, lr, decay, partials, (const sj_sgd_step*)nullptr,
-                     (const double*)nullptr);
+  launch_factored((hipStream_t)stream, meta, tiles, action, lr, decay, partials, nullptr, nullptr);
   SJ_LAUNCH_CHECK(action == 1 ? "parameter_gradient_update"
                               : action == 0 ? "parameter_gradient_materialize" : "parameter_gradient_norm");
   return SJ_OK;
@@ -957,8 +981,7 @@ extern "C" int sj_factored_apply(void* stream, const void* meta, long tiles, int
 int sjh::factored_update_staged(hipStream_t stream, const void* meta, long tiles, const sj_sgd_step* step,
                                 const double* sumsq) {
   SJ_REQUIRE(meta && step && tiles > 0 && tiles < (1L << 31), "compact SGD update: arguments");
-  hipLaunchKernelGGL(k_factored_apply, dim3((unsigned)tiles), dim3(256), 0, stream, (const uint8_t*)meta, 1, 0.f,
-                     0.f, (double*)nullptr, step, sumsq);
+  launch_factored(stream, meta, tiles, 1, 0.f, 0.f, nullptr, step, sumsq);
   SJ_LAUNCH_CHECK("parameter_gradient_update");
   return SJ_OK;
 }

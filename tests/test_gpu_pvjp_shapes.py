@@ -87,3 +87,28 @@ def test_coefficient_tiles(N, rows, b, n):
                                ws.p if ws_bytes else None, ws_bytes)
         sync()
         assert rel(C.host(), (eh + el) @ (dh + dl)) < 3e-5
+
+
+@pytest.mark.parametrize("a,b,R", [(16383, 40, 5), (16400, 40, 5), (16401, 37, 9)])
+def test_factored_apply_table_sizes(N, a, b, R):
+    """1024 tiles (the latency form's last table) and more (the wide form's), ragged rows, columns and rank."""
+    rng = np.random.default_rng(a + b)
+    f = lambda *s: rng.normal(0, 1, s).astype(np.float32)
+    left, right, tail, w = f(a, R), f(R, b), f(3, b), f(a, b)
+    fmap = np.full(a, -1, np.int32)
+    fmap[[0, 17, a - 1]] = [2, 0, 1]
+    L, RT, TL, MP, W = dev(left), dev(right), dev(tail), dev(fmap, "i32"), dev(w)
+    TA = (N.FactoredTerm * 1)(N.FactoredTerm(L.ptr, RT.ptr, TL.ptr, MP.ptr, R, 0.5, b))
+    PA = (N.FactoredParam * 1)(N.FactoredParam(W.ptr, None, a, b, 1, 0, 1, b, None))
+    nb = N.load().sj_factored_meta_bytes(PA, 1, 1)
+    host, tiles = np.zeros(nb, np.uint8), ctypes.c_long()
+    N.api.sj_factored_pack(PA, 1, TA, 1, ctypes.c_void_p(host.ctypes.data), nb, ctypes.byref(tiles))
+    assert tiles.value == -(-a // 16)
+    meta, part = dev(host, "u8"), empty(tiles.value, "f64")
+    N.api.sj_factored_apply(None, meta.p, tiles.value, 2, cf(0), cf(0), part.p)
+    N.api.sj_factored_apply(None, meta.p, tiles.value, 1, cf(0.25), cf(0.125), None)
+    sync()
+    g = 0.5 * left.astype(np.float64) @ right
+    g[[0, 17, a - 1]] += 0.5 * tail[[2, 0, 1]].astype(np.float64)
+    assert rel(part.host().sum(), (g ** 2).sum()) < 1e-6  # fp32 sums of R terms
+    assert rel(W.host().reshape(a, b), w * 0.875 - 0.25 * g) < 1e-6

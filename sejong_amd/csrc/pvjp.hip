@@ -78,9 +78,12 @@ __device__ __forceinline__ bool parallel_picks(uint64_t state, long size, int co
 }
 
 // parameter_indices (parameter.py:25-62).  One workgroup.  Up to 64 columns
-// and 64 blocks: the picks as above (17 -> 8 us at 2752 donor columns,
+// and 64 blocks: the picks as above (15 -> 5 us at 2752 donor columns,
 // 16 + 4 picks: the serial form below is a chain of dependent memory accesses
-// and 64-bit remainders), then the rows and the map by all lanes.  Otherwise
+// and 64-bit remainders), then the rows, and the map cleared and scattered
+// from them, by all lanes (searching the blocks for each map entry instead
+// took 111 us at 26 blocks of 64 in 16384 rows and 890 at 60 of 32 in 65536,
+// this 10 and 20).  Otherwise
 // the scratch permutations are initialised in parallel and the draws run
 // serially in lane 0.
 __global__ __launch_bounds__(256) void k_pvjp_indices(int32_t* __restrict__ scratch, int32_t* __restrict__ columns,
@@ -102,15 +105,13 @@ __global__ __launch_bounds__(256) void k_pvjp_indices(int32_t* __restrict__ scra
     }
     __syncthreads();
     if (fast) {
+      for (long i = t; i < A; i += 256) map[i] = -1;
+      __syncthreads();
       for (long p = t; p < S * group; p += 256) {
         const long index = block[p / group] * group + p % group;
-        rows[p] = index < A ? (int32_t)index : -1;
-      }
-      for (long i = t; i < A; i += 256) {
-        const long blk = i / group;
-        int32_t m = -1;
-        for (int q = 0; q < S; q++) m = block[q] == blk ? (int32_t)(q * group + i % group) : m;
-        map[i] = m;
+        const bool in = index < A;
+        rows[p] = in ? (int32_t)index : -1;
+        if (in) map[index] = (int32_t)p;
       }
       return;
     }

@@ -8,7 +8,7 @@ import pytest
 
 from oracle import oracle as O
 from oracle import pvjp as P
-from tests.gpu_util import dev, empty, rel, rnd, sync, zeros
+from tests.gpu_util import best_us, dev, empty, rel, rnd, sync, zeros
 
 pytestmark = pytest.mark.gpu
 cf = ctypes.c_float
@@ -36,6 +36,20 @@ def test_indices_match_the_reference_draws(N, A, B, block, S, R, seed):
     np.testing.assert_array_equal(cols.host(), c)
     np.testing.assert_array_equal(rows.host(), r)
     np.testing.assert_array_equal(fmap.host(), m)
+
+
+def test_indices_of_many_blocks_in_one_pass(N):
+    """The map is one pass over its rows whatever the blocks (60 of them once
+    took 10 times as long as one; the draws themselves are a few us)."""
+    A, B, block, R = 65536, 60000, 32, 8
+    NB = A // block
+    scr, cols, fmap = zeros(B + NB, "i32"), zeros(R, "i32"), zeros(A, "i32")
+
+    def us(S):
+        rows = zeros(S * block, "i32")
+        return best_us(lambda: N.api.sj_pvjp_indices(None, ctypes.c_uint64(3), A, B, NB, S, R, block, scr.p, cols.p,
+                                                     rows.p, fmap.p))
+    assert us(60) < 2.5 * us(1)
 
 
 @pytest.mark.parametrize("n,R,dt,dup", [(64, 1, "f32", False), (65, 16, "bf16", False), (1000, 17, "f32", False),

@@ -323,7 +323,7 @@ __global__ __launch_bounds__(64) void k_chol_inv(const double* __restrict__ gram
     const double d = lane_f64(g[c], c);
     const bool kp = d > e2 * lane_f64(dg, c) && d > 0.0;
     const double iv = kp ? 1.0 / sqrt(d) : 0.0;
-    const double v = t > c ? g[c] * iv : 0.0;
+    const double v = kp && t > c ? g[c] * iv : 0.0;
     inv = t == c ? iv : inv;
     g[c] = v;
 #pragma unroll
@@ -335,7 +335,8 @@ __global__ __launch_bounds__(64) void k_chol_inv(const double* __restrict__ gram
     double v = t == j ? 1.0 : 0.0;
 #pragma unroll
     for (int k = 0; k < j; k++) v = fma(-lane_f64(g[k], j), tr[k], v);
-    tr[j] = v * lane_f64(inv, j);  // a dropped column's reciprocal is 0
+    const double iv = lane_f64(inv, j);
+    tr[j] = iv > 0.0 ? v * iv : 0.0;  // 0: a dropped column
     if (t < R && j < R) tmat[t * R + j] = (float)tr[j];
   }
 }

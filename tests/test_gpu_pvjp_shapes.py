@@ -80,6 +80,23 @@ def test_basis_orthonormal_span_and_drop(N, n, R, dt, dup):
     assert rel(Q[:, :keep] @ (Q[:, :keep].T @ V), Qr @ (Qr.T @ V)) < 2e-6
 
 
+@pytest.mark.parametrize("R,bad", [(5, 0), (16, 7), (20, 19), (64, 33)])
+def test_basis_value_out_of_range_stays_in_its_row(N, R, bad):
+    """A column with an infinite value is dropped (its pivot is not finite):
+    the other rows of Q stay finite whatever the column's place."""
+    n = 300
+    y = rnd((n, R), "f32", np.random.default_rng(R))
+    y[41, bad] = np.inf
+    cols, q = np.arange(R, dtype=np.int32), empty(n * R)
+    lib = N.load()
+    wb = lib.sj_pvjp_basis_workspace_bytes(n, R)
+    ws = empty(wb, "u8")
+    N.api.sj_pvjp_basis(None, dev(y, "f32").p, 0, R, n, dev(cols, "i32").p, R, cf(lib.sj_pvjp_basis_tolerance(n, R)),
+                        q.p, ws.p, wb)
+    sync()
+    assert np.isfinite(np.delete(q.host().reshape(n, R), 41, axis=0)).all()
+
+
 @pytest.mark.parametrize("rows,b,n", [(48, 200, 8192), (80, 136, 8200), (112, 64, 8192), (144, 264, 8256),
                                       (176, 72, 16384), (272, 320, 8192), (145, 8, 9000)])
 def test_coefficient_tiles(N, rows, b, n):

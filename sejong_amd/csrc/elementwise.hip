@@ -451,35 +451,39 @@ extern "C" int sj_embedding_fwd(void* stream, const void* w, int wd, const int32
 
 extern "C" size_t sj_embedding_bwd_workspace_bytes(long n, long vocab) { return 0; }
 
-// Faster form for d % 4 == 0 (16-byte rows): workgroup (v, c) owns columns
-// 128 c .. + 127 of vocabulary row v.  Each round scans 16 ids per thread
+// Faster form for d % 4 == 0 (16-byte rows): workgroup (v, c) owns CPW column
+// chunks of EMB_COLS of vocabulary row v.  Each round scans 16 ids per thread
 // (4096 tokens) and compacts the matches in token order with one block scan;
-// then the matching rows come in batches of 64, eight 16-byte loads per
-// thread in flight into LDS while the batch before is added, column by
+// then, chunk by chunk, the matching rows come in batches of BATCH, their
+// 16-byte loads in flight into LDS while the batch before is added, column by
 // column in token order (the same order, hence the same bits, as
-// k_embedding_bwd).  Bound by the longest row of a skewed batch: one load in
-// flight per thread and column took 31 us with 256 of 4096 tokens alike (d
-// 384), now 10.
-constexpr int EMB_IDS = 16, EMB_COLS = 128, EMB_BATCH = 64;
+// k_embedding_bwd).  Bound by the longest row of a skewed batch (one load in
+// flight per thread and column took 20 us at 257 rows, 4096 tokens, d 384,
+// now 9), and with a large vocabulary by the id scans of the rows without a
+// match, which leave after one barrier.
+constexpr int EMB_IDS = 16, EMB_COLS = 128;
 // sq (nullable): FP64 sum of squares of the columns this workgroup stores, at
 // sq[its linear index] (the gradient-norm hook)
-__global__ __launch_bounds__(EMB_THREADS) void k_embedding_bwd4(const float* __restrict__ dy,
-                                                                const int32_t* __restrict__ ids,
-                                                                float* __restrict__ dw, long n, long d, double* sq) {
-  constexpr int W = EMB_THREADS * EMB_IDS, SLOTS = EMB_THREADS / (EMB_COLS / 4), PER = EMB_BATCH / SLOTS;
+template <int CPW, int BATCH, int MINW>
+__global__ __launch_bounds__(EMB_THREADS, MINW) void k_embedding_bwd4(const float* __restrict__ dy,
+                                                                      const int32_t* __restrict__ ids,
+                                                                      float* __restrict__ dw, long n, long d,
+                                                                      double* sq) {
+  constexpr int W = EMB_THREADS * EMB_IDS, SLOTS = EMB_THREADS / (EMB_COLS / 4), PER = BATCH / SLOTS;
   __shared__ uint16_t matches[W];
-  __shared__ int wave_total[EMB_THREADS / 64];
-  __shared__ __attribute__((aligned(16))) float rows[EMB_BATCH * EMB_COLS];
+  __shared__ int wave_total[2][EMB_THREADS / 64];  // of this round and of the one before
+  __shared__ __attribute__((aligned(16))) float rows[BATCH * EMB_COLS];
   const int v = blockIdx.x;
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const long col0 = (long)blockIdx.y * EMB_COLS;
-  // loading: 16-byte chunk lc of batch rows slot, slot + SLOTS, ...; adding: column t of the chunk
+  const long colw = (long)blockIdx.y * CPW * EMB_COLS;
+  // loading: 16-byte chunk lc of batch rows slot, slot + SLOTS, ...; adding: column t of a chunk
   const int lc = t % (EMB_COLS / 4), slot = t / (EMB_COLS / 4);
-  const bool lok = col0 + 4 * lc < d, aok = t < EMB_COLS && col0 + t < d;
-  const float* src = dy + col0 + 4 * lc;
   const bool ivec = ((uintptr_t)ids & 15) == 0;
-  float acc = 0.f;
-  for (long base = 0; base < n; base += W) {
+  float acc[CPW];
+#pragma unroll
+  for (int c = 0; c < CPW; c++) acc[c] = 0.f;
+  int round = 0;
+  for (long base = 0; base < n; base += W, round ^= 1) {
     const long i0 = base + (long)t * EMB_IDS;
     uint32_t hit = 0;
     if (ivec && i0 + EMB_IDS <= n) {
@@ -496,19 +500,22 @@ __global__ __launch_bounds__(EMB_THREADS) void k_embedding_bwd4(const float* __r
     }
     const int cnt = __popc(hit);
     int incl = cnt;  // inclusive scan over the wave
+    if (__any(hit != 0)) {
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += y;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
+      }
     }
-    if (lane == 63) wave_total[w] = incl;
+    if (lane == 63) wave_total[round][w] = incl;
     __syncthreads();
     int before = 0, total = 0;
 #pragma unroll
     for (int j = 0; j < EMB_THREADS / 64; j++) {
-      if (j < w) before += wave_total[j];
-      total += wave_total[j];
+      if (j < w) before += wave_total[round][j];
+      total += wave_total[round][j];
     }
+    if (total == 0) continue;  // uniform
     int pos = before + incl - cnt;
     while (hit) {
       const int k = __ffs(hit) - 1;
@@ -516,35 +523,56 @@ __global__ __launch_bounds__(EMB_THREADS) void k_embedding_bwd4(const float* __r
       matches[pos++] = (uint16_t)(t * EMB_IDS + k);
     }
     __syncthreads();
-    float4 r[PER];
-    auto load = [&](int m0) {
 #pragma unroll
-      for (int i = 0; i < PER; i++) {
-        const int m = m0 + slot + SLOTS * i;
-        r[i] = lok && m < total ? *(const float4*)(src + (base + matches[m]) * d) : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-    };
-    if (total > 0) load(0);
-    for (int m0 = 0; m0 < total; m0 += EMB_BATCH) {
+    for (int c = 0; c < CPW; c++) {
+      const long col0 = colw + c * EMB_COLS;
+      if (col0 >= d) break;  // uniform
+      const bool lok = col0 + 4 * lc < d;
+      const float* src = dy + col0 + 4 * lc;
+      float4 r[PER];
+      auto load = [&](int m0) {
 #pragma unroll
-      for (int i = 0; i < PER; i++) *(float4*)(rows + (slot + SLOTS * i) * EMB_COLS + 4 * lc) = r[i];
-      __syncthreads();
-      if (m0 + EMB_BATCH < total) load(m0 + EMB_BATCH);
-      if (aok) {
-        const int cntb = total - m0 < EMB_BATCH ? total - m0 : EMB_BATCH;
+        for (int i = 0; i < PER; i++) {
+          const int m = m0 + slot + SLOTS * i;
+          r[i] = lok && m < total ? *(const float4*)(src + (base + matches[m]) * d) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+      };
+      load(0);
+      for (int m0 = 0; m0 < total; m0 += BATCH) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) *(float4*)(rows + (slot + SLOTS * i) * EMB_COLS + 4 * lc) = r[i];
+        __syncthreads();
+        if (m0 + BATCH < total) load(m0 + BATCH);
+        if (t < EMB_COLS && col0 + t < d) {
+          const int cntb = total - m0 < BATCH ? total - m0 : BATCH;
 #pragma unroll 8
-        for (int m = 0; m < cntb; m++) acc += rows[m * EMB_COLS + t];
+          for (int m = 0; m < cntb; m++) acc[c] += rows[m * EMB_COLS + t];
+        }
+        __syncthreads();
       }
-      __syncthreads();
     }
-    __syncthreads();
   }
-  if (aok) dw[(long)v * d + col0 + t] = acc;
+  double q = 0.0;
+#pragma unroll
+  for (int c = 0; c < CPW; c++) {
+    const long col = colw + c * EMB_COLS + t;
+    if (t < EMB_COLS && col < d) {
+      dw[(long)v * d + col] = acc[c];
+      q += (double)acc[c] * acc[c];
+    }
+  }
   if (sq) {
     __shared__ double qred[EMB_THREADS / 64];
-    const double q = block_sum<double, EMB_THREADS>(aok ? (double)acc * acc : 0.0, qred);
+    q = block_sum<double, EMB_THREADS>(q, qred);
     if (t == 0) sq[blockIdx.x + gridDim.x * blockIdx.y] = q;
   }
+}
+
+template <int CPW, int BATCH, int MINW>
+void embedding_bwd4(hipStream_t s, const float* dy, const int32_t* ids, float* dw, long n, long d, long vocab) {
+  const long parts = (d + CPW * EMB_COLS - 1) / (CPW * EMB_COLS);
+  hipLaunchKernelGGL((k_embedding_bwd4<CPW, BATCH, MINW>), dim3((unsigned)vocab, (unsigned)parts), dim3(EMB_THREADS), 0, s,
+                     dy, ids, dw, n, d, sjh::grad_sq().take(vocab * parts));
 }
 
 extern "C" int sj_embedding_bwd(void* stream, const float* dy, const int32_t* ids, float* dw, long n, long d,
@@ -552,9 +580,21 @@ extern "C" int sj_embedding_bwd(void* stream, const float* dy, const int32_t* id
   SJ_REQUIRE(n >= 0 && d > 0 && d <= 8 * EMB_THREADS && vocab > 0, "embedding_backward: n %ld d %ld vocab %ld", n,
              d, vocab);
   if (d % 4 == 0 && d <= 8 * EMB_THREADS && ((uintptr_t)dy & 15) == 0 && ((uintptr_t)dw & 15) == 0) {
-    const long chunks = (d + EMB_COLS - 1) / EMB_COLS;
-    hipLaunchKernelGGL(k_embedding_bwd4, dim3((unsigned)vocab, (unsigned)chunks), dim3(EMB_THREADS), 0,
-                       (hipStream_t)stream, dy, ids, dw, n, d, sjh::grad_sq().take(vocab * chunks));
+    // One chunk a workgroup splits a skewed batch's longest row best, but every
+    // workgroup scans all ids and few fit on a CU (41 KB of LDS): it serves until
+    // the workgroups are some rounds of the chip (fewer with few tokens, whose
+    // rows are short), then two chunks, then four.  us at 1 / 2 / 4 chunks:
+    // 257 rows, 4096 tokens, d 384 9.2 / 14.7 / 31; 1024 rows, d 1024 27 / 15 /
+    // 26; 2048 rows, 512 tokens, d 384 16 / 7.6 / 5.6; 32768 rows, 4096 tokens,
+    // d 1024 422 / 142 / 76.
+    const long cu = 256, chunks = (d + EMB_COLS - 1) / EMB_COLS;
+    hipStream_t s = (hipStream_t)stream;
+    if (vocab * chunks <= (n > 1024 ? 9 : 4) * cu)
+      embedding_bwd4<1, 64, 3>(s, dy, ids, dw, n, d, vocab);
+    else if (vocab * ((chunks + 1) / 2) <= (n > 1024 ? 32 : 8) * cu)
+      embedding_bwd4<2, 32, 6>(s, dy, ids, dw, n, d, vocab);
+    else
+      embedding_bwd4<4, 16, 8>(s, dy, ids, dw, n, d, vocab);
   } else {
     hipLaunchKernelGGL(k_embedding_bwd, dim3((unsigned)vocab), dim3(EMB_THREADS), 0, (hipStream_t)stream, dy, ids, dw,
                        n, d);

@@ -1346,21 +1346,22 @@ void launch_rows(hipStream_t s, const RowArgs& a, long heads) {
 // Raise the dynamic-LDS limit of the kernels that stage more than 64 KB
 // (head_dim above 64) once, outside any capture.
 int rows_prepare() {
-  static int done = 0, status = SJ_OK;
-  if (done) return status;
-  done = 1;
-  auto set = [&](rt_kernel k, int, size_t lds) {
-    if (status) return;
-    const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) status = sjh::hip_check(e, "attention rows: LDS attribute");
-  };
-  for (long rows : {1L, 1L << 20}) {
-    rt_pick<RtFwd>(128, rows, set);
-    rt_pick<RtCached>(128, rows, set);
-    rt_pick<RtDq>(128, rows, set);
-    rt_pick<RtDkv>(128, rows, set);
-  }
-  return status;
+  static sj::OncePerDevice once;
+  return sjh::once_per_device(once, [] {
+    int status = SJ_OK;
+    auto set = [&](rt_kernel k, int, size_t lds) {
+      if (status) return;
+      const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) status = sjh::hip_check(e, "attention rows: LDS attribute");
+    };
+    for (long rows : {1L, 1L << 20}) {
+      rt_pick<RtFwd>(128, rows, set);
+      rt_pick<RtCached>(128, rows, set);
+      rt_pick<RtDq>(128, rows, set);
+      rt_pick<RtDkv>(128, rows, set);
+    }
+    return status;
+  });
 }
 
 bool use_mfma(int dtype, long head_dim, long window, long t, long ldq, long ldk, long ldv, long ldo,

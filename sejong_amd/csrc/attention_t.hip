@@ -1271,24 +1271,23 @@ extern "C" int sj_attention_bwd_plan(long t, long window, long pairs, int cus, u
 }
 
 int sjh::attention_t_prepare() {
-  static int done = 0, status = SJ_OK;
-  if (done) return status;
-  done = 1;
-  hipError_t e = hipFuncSetAttribute((const void*)k_attn2_fwd<NS_FWD>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_FWD);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_attn2_fwd_cached<NS_FWD>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)LDS_FWD);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_attn2_bwd, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BWD);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_attn2_bwd_dq, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DQ);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_attn2_bwd_dkv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DKV);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_attn2_bwd_g<GROUPED_G>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)(LDS_BWD_G + 16));
-  status = e == hipSuccess ? SJ_OK : sjh::hip_check(e, "attention: LDS attribute");
-  return status;
+  static sj::OncePerDevice once;
+  return once_per_device(once, [] {
+    hipError_t e = hipFuncSetAttribute((const void*)k_attn2_fwd<NS_FWD>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_FWD);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void*)k_attn2_fwd_cached<NS_FWD>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)LDS_FWD);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void*)k_attn2_bwd, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BWD);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void*)k_attn2_bwd_dq, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DQ);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void*)k_attn2_bwd_dkv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DKV);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void*)k_attn2_bwd_g<GROUPED_G>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)(LDS_BWD_G + 16));
+    return e == hipSuccess ? (int)SJ_OK : sjh::hip_check(e, "attention: LDS attribute");
+  });
 }
 
 static int check_t(const void* qkv, long ldqkv, long ldt, long batch, long t, long hq, long hk, long head_dim,

@@ -8,6 +8,7 @@
 #include <stddef.h>
 
 #include "../../include/sejong_hip.h"
+#include "once.h"
 
 namespace sj {
 
@@ -243,6 +244,14 @@ GradSq& grad_sq();
 // Record a failure message for sj_last_error() and return the status.
 int fail(int status, const char* fmt, ...);
 int hip_check(hipError_t e, const char* what);
+// f's status (SJ_OK or a failure), run once on each device: the kernel
+// attributes f sets belong to the current device
+template <class F>
+int once_per_device(sj::OncePerDevice& once, F f) {
+  int device = 0;
+  const hipError_t e = hipGetDevice(&device);
+  return e == hipSuccess ? once(device, f) : hip_check(e, "current device");
+}
 // sj_rmsnorm_bwd_p with the dw reduce left to rmsnorm_reduce_multi (partial:
 // sj_rmsnorm_bwd_p_workspace_bytes of its own)
 int rmsnorm_bwd_p_deferred(void* stream, const uint16_t* x, const uint16_t* w, const float* dy, const float* dx_acc,

@@ -2034,34 +2034,34 @@ int set_attrs_kw() {
 // stream capture); called by sj_model_create and lazily by the entry points.
 namespace sjh {
 int gemm_fast_prepare() {
-  static int done = 0, status = SJ_OK;
-  if (done) return status;
-  done = 1;
-  status = set_attrs_planes<E_STORE>();
-  if (!status) status = set_attrs_planes<E_PARTIAL>();
-  if (!status) status = set_attrs_planes<E_QKV>();
-  if (!status) status = set_attrs_planes<E_RESID>();
-  if (!status) status = set_attrs_planes<E_GATEUP>();
-  if (!status) status = set_attrs_planes<E_SWIGLU_BWD>();
-  if (!status) status = set_attrs_planes<E_SWIGLU_ROWS>();
-  if (!status) status = set_attrs_planes<E_PLANES>();
-  if (!status) status = set_attrs_planes<E_STORE, 3>();
-  if (!status) status = set_attrs_planes<E_PARTIAL, 3>();
-  if (!status) status = set_attrs_tiles<E_STORE, 1, 2, 1>();
-  if (!status) status = set_attrs_tiles<E_PARTIAL, 1, 2, 1>();
-  if (!status) status = set_attrs_tiles<E_STORE, 2, 2, 2>();
-  if (!status) status = set_attrs_tiles<E_PARTIAL, 2, 2, 2>();
-  if (!status) status = set_attr_pp<2, 1, E_STORE, 0>();
-  if (!status) status = set_attr_pp<1, 1, E_RESID, 0>();
-  if (!status) status = set_attr_pp<1, 1, E_GATEUP, 0>();
-  if (!status) status = set_attr_pp<2, 1, E_PLANES, 0>();
-  if (!status) status = set_attr_pp<1, 2, E_STORE, 3>();
-  if (!status) status = set_attr_pp<1, 2, E_PARTIAL, 3>();
-  if (!status) status = set_attrs_tall<E_STORE>();
-  if (!status) status = set_attrs_tall<E_PARTIAL>();
-  if (!status) status = set_attrs_kw<E_STORE>();
-  if (!status) status = set_attrs_kw<E_PARTIAL>();
-  return status;
+  static sj::OncePerDevice once;
+  return once_per_device(once, [] {
+    int status = set_attrs_planes<E_STORE>();
+    if (!status) status = set_attrs_planes<E_PARTIAL>();
+    if (!status) status = set_attrs_planes<E_QKV>();
+    if (!status) status = set_attrs_planes<E_RESID>();
+    if (!status) status = set_attrs_planes<E_GATEUP>();
+    if (!status) status = set_attrs_planes<E_SWIGLU_BWD>();
+    if (!status) status = set_attrs_planes<E_SWIGLU_ROWS>();
+    if (!status) status = set_attrs_planes<E_PLANES>();
+    if (!status) status = set_attrs_planes<E_STORE, 3>();
+    if (!status) status = set_attrs_planes<E_PARTIAL, 3>();
+    if (!status) status = set_attrs_tiles<E_STORE, 1, 2, 1>();
+    if (!status) status = set_attrs_tiles<E_PARTIAL, 1, 2, 1>();
+    if (!status) status = set_attrs_tiles<E_STORE, 2, 2, 2>();
+    if (!status) status = set_attrs_tiles<E_PARTIAL, 2, 2, 2>();
+    if (!status) status = set_attr_pp<2, 1, E_STORE, 0>();
+    if (!status) status = set_attr_pp<1, 1, E_RESID, 0>();
+    if (!status) status = set_attr_pp<1, 1, E_GATEUP, 0>();
+    if (!status) status = set_attr_pp<2, 1, E_PLANES, 0>();
+    if (!status) status = set_attr_pp<1, 2, E_STORE, 3>();
+    if (!status) status = set_attr_pp<1, 2, E_PARTIAL, 3>();
+    if (!status) status = set_attrs_tall<E_STORE>();
+    if (!status) status = set_attrs_tall<E_PARTIAL>();
+    if (!status) status = set_attrs_kw<E_STORE>();
+    if (!status) status = set_attrs_kw<E_PARTIAL>();
+    return status;
+  });
 }
 }  // namespace sjh
 

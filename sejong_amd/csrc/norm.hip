@@ -500,19 +500,18 @@ hipError_t set_np_attrs() {
 
 namespace sjh {
 int norm_prepare() {
-  static int done = 0, status = SJ_OK;
-  if (done) return status;
-  done = 1;
-  hipError_t e = set_np_attrs<1>();
-  if (e == hipSuccess) e = set_np_attrs<2>();
-  if (e == hipSuccess) e = set_np_attrs<3>();
-  if (e == hipSuccess) e = set_np_attrs<4>();
-  if (e == hipSuccess) e = set_np_attrs<5>();
-  if (e == hipSuccess) e = set_np_attrs<6>();
-  if (e == hipSuccess) e = set_np_attrs<7>();
-  if (e == hipSuccess) e = set_np_attrs<8>();
-  status = e == hipSuccess ? SJ_OK : sjh::hip_check(e, "rmsnorm: LDS attribute");
-  return status;
+  static sj::OncePerDevice once;
+  return once_per_device(once, [] {
+    hipError_t e = set_np_attrs<1>();
+    if (e == hipSuccess) e = set_np_attrs<2>();
+    if (e == hipSuccess) e = set_np_attrs<3>();
+    if (e == hipSuccess) e = set_np_attrs<4>();
+    if (e == hipSuccess) e = set_np_attrs<5>();
+    if (e == hipSuccess) e = set_np_attrs<6>();
+    if (e == hipSuccess) e = set_np_attrs<7>();
+    if (e == hipSuccess) e = set_np_attrs<8>();
+    return e == hipSuccess ? (int)SJ_OK : sjh::hip_check(e, "rmsnorm: LDS attribute");
+  });
 }
 }  // namespace sjh
 

@@ -182,7 +182,7 @@ int attention_fwd_cached_t(void* stream, const uint16_t* q, long ldq, const uint
 // project_qkv + RoPE (rows from x, or the embedding rows of the host's ids,
 // then also written to xout), projection + residual, RMSNorm + gate/up +
 // SwiGLU (h only), final RMSNorm + head on one row; the bits of the tiled ones
-constexpr int DECODE_ROWS = 16;
+constexpr int DECODE_ROWS = 8;
 bool decode_rows_ok(long n, long d);
 int decode_qkv(hipStream_t s, const uint16_t* x, const uint16_t* table, const int32_t* ids, uint16_t* xout,
                const uint16_t* wn, float eps, long n, long d, const uint16_t* wqkv_t, long kv, uint16_t* q, uint16_t* k,

@@ -1,6 +1,6 @@
 // The blocks' products for a few rows: the KV-cache path's decode steps
 // (Model::forward_cached, model lib.rs:362-372; architecture.rs:474-533) and
-// chunks of up to 16 tokens, bf16.
+// chunks of up to 8 tokens, bf16.
 //
 // A tiled product gives a row-starved call N / 64 workgroups that each stream
 // 64 weight rows through LDS stages behind barriers: at one token (d 384)
@@ -12,7 +12,14 @@
 // from cache) and leaves the normed rows in LDS, so a layer is five launches
 // instead of seven and no normed row travels through memory.  The bound is
 // one weight read's latency plus the launch.  25 calls (a prompt of 200 and
-// 24 tokens, 6 layers, d 384): 7.2 -> 4.8 ms (the rest is launches: 32 a token, about 4 us of host time each, one read-back).
+// 24 tokens, 6 layers, d 384): 7.2 -> 4.8 ms (the rest is launches: 32 a token,
+// about 4 us of host time each, one read-back).
+//
+// The rows' norms run one after another in every wave, so each further row
+// adds a latency per product where the tiled path's time stays: a call of
+// 1 / 4 / 8 / 12 / 16 tokens takes 158 / 206 / 255 / 305 / 350 us (6 layers,
+// d 384; tiled 272 / 272 / 279 / 291 / 297) and 423 / 548 / 680 / 808 / 930
+// (12 layers, d 1024; tiled 763 / 786 / 806 / 830 / 847).  Hence 8 rows.
 //
 // Every product keeps the k order, the MFMA shape and the roundings of the
 // tiled one (k_gemm_fast, k_rms_fwd_t), so the logits keep their bits: a
@@ -25,7 +32,7 @@ using namespace sj;
 
 namespace {
 
-constexpr int DR = sjh::DECODE_ROWS;  // rows of one MFMA tile
+constexpr int DR = sjh::DECODE_ROWS;  // at most the 16 of one MFMA tile
 constexpr int U = 8;                  // k-steps (32) per register group, two groups in flight
 enum { D_QKV = 0, D_RESID = 1, D_GATEUP = 2, D_HEAD = 3 };
 

@@ -2905,7 +2905,7 @@ int calloc_(sj_cache* c, void** p, size_t bytes) {
 // new rows in c->x[0] at positions L .. L + n - 1 of the stage's cache;
 // then the stage's closing norm into `out` (the encoder, global or decoder
 // norm, or the final norm of a one-stage model; null: *last receives the
-// blocks' output rows instead).  Up to 16 rows run the few-row products
+// blocks' output rows instead).  Up to 8 rows run the few-row products
 // (decode.hip); `tokens` (host, nullable, few rows only): the first layer's
 // rows are these tokens' embeddings, not c->x[0].
 int cached_blocks(sj_model* m, sj_cache* c, int si, long n, long L, void* out, const int32_t* tokens = nullptr,
@@ -2946,13 +2946,13 @@ int cached_blocks(sj_model* m, sj_cache* c, int si, long n, long L, void* out, c
     if (m->planes) {
       const uint16_t *W = m->mirror, *WT = m->mirror_t;
       if (!few) {
-      TRY(sj_rmsnorm_fwd_t(s, (const uint16_t*)x, W + y.an, (uint16_t*)c->z, nullptr, 0, n, d, eps));
-      TRY(sjh::qkv_fwd_t_out(s, (const uint16_t*)c->z, d, n, d, WT + y.qkv, d, d, J, (uint16_t*)c->q, d,
-                             (uint16_t*)kc, J, (uint16_t*)vc, J, rope, rope_t, S.Dh, nullptr, 0));
-      TRY(sj_attention_fwd_cached(s, c->q, d, c->keys[l], c->values[l], J, cap, dt, n, L, S.HQ, S.HK, S.Dh, S.window,
-                                  c->o, d));
-      TRY(sj_linear_residual_fwd_t(s, (const uint16_t*)c->o, d, n, d, WT + y.wo, d, d, (const uint16_t*)x, d,
-                                   (uint16_t*)c->x1, d));
+        TRY(sj_rmsnorm_fwd_t(s, (const uint16_t*)x, W + y.an, (uint16_t*)c->z, nullptr, 0, n, d, eps));
+        TRY(sjh::qkv_fwd_t_out(s, (const uint16_t*)c->z, d, n, d, WT + y.qkv, d, d, J, (uint16_t*)c->q, d,
+                               (uint16_t*)kc, J, (uint16_t*)vc, J, rope, rope_t, S.Dh, nullptr, 0));
+        TRY(sj_attention_fwd_cached(s, c->q, d, c->keys[l], c->values[l], J, cap, dt, n, L, S.HQ, S.HK, S.Dh, S.window,
+                                    c->o, d));
+        TRY(sj_linear_residual_fwd_t(s, (const uint16_t*)c->o, d, n, d, WT + y.wo, d, d, (const uint16_t*)x, d,
+                                     (uint16_t*)c->x1, d));
       }
       TRY(sj_rmsnorm_fwd_t(s, (const uint16_t*)c->x1, W + y.fn, (uint16_t*)c->z2, nullptr, 0, n, d, eps));
       if (m->E) {  // routed experts over the new rows (architecture.rs:516-529)

@@ -222,6 +222,17 @@ int sj_down_bwd_swiglu(void *stream, const float *dy, long lddy, long M, long D,
  * Split-K through `workspace`
  * (sj_gemm_planes_workspace_bytes) with a fixed-order reduction. */
 size_t sj_gemm_planes_workspace_bytes(long M, long N, long K);
+/* Inspection of the products' dispatch (no counterpart in the reference: it is
+ * this library's scheduling, exposed for its tests; 256 CUs are assumed where
+ * there is no device).  op 0: sj_gemm_planes with A in two planes; 1:
+ * sj_gemm_planes_tn with Y in two planes; 2: sj_gate_up_fwd_t (N: ffn width);
+ * 3: sj_linear_residual_fwd_t; 4: sj_gemm_planes_split_out; 5: the parameter
+ * VJP's coefficient product (both operands in two planes, the second in row
+ * layout).  Outputs and workspace of any alignment and size the rules ask for.
+ * Sets the tile and the K slices (before rounding to whole steps) and returns
+ * the kernel: 0 k_gemm_fast, 1 k_gemm_kw (token-split dW), 2 k_gemm_pp
+ * (ping-pong), or a negative status. */
+int sj_gemm_planes_plan(int op, long M, long N, long K, int *bm, int *bn, int *splits);
 int sj_gemm_planes(void *stream, long M, long N, long K, const uint16_t *a_hi, const uint16_t *a_lo,
                    long lda, const uint16_t *b_hi, const uint16_t *b_lo, long ldb, void *c, int c_dtype,
                    long ldc, int accumulate, void *workspace, size_t workspace_bytes);

@@ -147,6 +147,7 @@ SIGNATURES = {
     "sj_linear_residual_fwd": (_I, [_P, _P, _L, _L, _L, _P, _L, _L, _P, _L, _P, _L, _I]),
     "sj_down_bwd_swiglu": (_I, [_P, _P, _L, _L, _L, _P, _L, _L, _P, _P, _L, _I, _P, _L]),
     "sj_gemm_planes_workspace_bytes": (_S, [_L, _L, _L]),
+    "sj_gemm_planes_plan": (_I, [_I, _L, _L, _L, _P, _P, _P]),
     "sj_gemm_planes": (_I, [_P, _L, _L, _L, _P, _P, _L, _P, _P, _L, _P, _I, _L, _I, _P, _S]),
     "sj_attention_fwd_tt": (_I, [_P, _P, _L, _L, _L, _L, _L, _L, _L, _L, _P, _L, _P, _P, _P, _L]),
     "sj_attention_bwd_tt_workspace_bytes": (_S, [_L, _L, _L, _L, _L]),
@@ -233,9 +234,10 @@ SIGNATURES = {
     "sj_model_buffer": (_I, [_P, ctypes.c_char_p, ctypes.POINTER(_P), ctypes.POINTER(_L)]),
 }
 
-# functions whose int result is a status (sj_attention_bwd_plan returns a count)
+# functions whose int result is a status (sj_attention_bwd_plan returns a
+# count, sj_gemm_planes_plan a kernel)
 STATUS_FUNCS = {n for n, (r, _) in SIGNATURES.items()
-                if r is _I and n not in ("sj_status_string", "sj_attention_bwd_plan")}
+                if r is _I and n not in ("sj_status_string", "sj_attention_bwd_plan", "sj_gemm_planes_plan")}
 
 _lib = None
 

@@ -24,6 +24,8 @@
 
 #include <hip/hip_ext.h>
 
+#include <initializer_list>
+
 #include "common.h"
 
 using namespace sj;
@@ -1757,7 +1759,7 @@ int splits_for(long M, long N, long K, int bm, int bn) {
 // split Y), so as many K slices as fill the CUs once, each at least 512
 // tokens.  SJ_GEMM_KW=0
 // selects the k_gemm_fast form; SJ_GEMM_KW_SPLITS=<n> overrides the slices
-// (sweeps).
+// (sweeps; with either set k_gemm_pp does not take the dW products).
 bool plan_kw(long M, long N, long K, int pa, int& splits) {
   static int on = -1, ov = 0;
   if (on < 0) {
@@ -1776,6 +1778,14 @@ bool plan_kw(long M, long N, long K, int pa, int& splits) {
   return true;
 }
 
+// Whether one of the sweep overrides is set: a rule steps aside for those of
+// the plan it would replace.
+bool overridden(std::initializer_list<const char*> names) {
+  for (const char* n : names)
+    if (getenv(n)) return true;
+  return false;
+}
+
 // Tiles of the parameter VJP's coefficient product (C = A Y, both operands
 // hi/lo planes, Y in row layout, few rows of A against long K).  It is bound
 // by the LDS DMA: a 64 x 64 tile stages 2 x (64 + 64) rows for 3 x 64 x 64
@@ -1787,7 +1797,8 @@ bool plan_kw(long M, long N, long K, int pa, int& splits) {
 // stages, and the partials' write and read.  144 x 5504 x 16384: 155 (64 x 64)
 // -> 107 us; 64-row tiles stay with the general plan.
 bool plan_tall(long M, long N, long K, int& bm, int& bn, int& splits) {
-  if (K < 8192 || M > 512) return false;
+  static const bool off = overridden({"SJ_GEMM_TILE", "SJ_GEMM_SPLITS", "SJ_GEMM_LK_TILE", "SJ_GEMM_LK_SPLITS"});
+  if (off || K < 8192 || M > 512) return false;
   const long cu = cus();
   double best = 0;
   int bs = 1, bbm = 0, bbn = 0;
@@ -1878,6 +1889,15 @@ int launch_planes_one(hipStream_t s, const FParams& p, int pa, int pb, int bm, i
 bool ok16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
 constexpr int PP_SPLITS = 8;  // K slices of a dW product at most
+// SJ_GEMM_PP=0 leaves every product to k_gemm_fast and k_gemm_kw (sweeps, and
+// the comparison of their bits); their own overrides do the same.
+bool pp_off() {
+  static const bool off = [] {
+    const char* e = getenv("SJ_GEMM_PP");
+    return (e && atoi(e) == 0) || overridden({"SJ_GEMM_TILE", "SJ_GEMM_SPLITS", "SJ_GEMM_STAGES"});
+  }();
+  return off;
+}
 // The ping-pong kernel's modelled time, us: rounds of one tile per CU, each a
 // fixed part (fill, epilogue) and stages of 32 k that take a0 + a1 x the share
 // of the CUs at work (the chip's matrix rate levels off near 1 PFLOP/s).
@@ -1900,6 +1920,7 @@ double pp_us(long t, double stages, double fixed, double a0, double a1) {
 // SwiGLU-derivative (16384 x 2752 x 1024: 298 -> 308) epilogues did not win
 // at any shape and stay with k_gemm_fast.
 bool pp_wins(int epi, long M, long N, long K) {
+  if (pp_off()) return false;
   const double mn = (double)M * (double)N, st = (double)K / PP_K, fl = 2.0 * mn * (double)K;
   double pp, old;
   if (epi == E_GATEUP) {
@@ -1925,7 +1946,9 @@ bool pp_wins(int epi, long M, long N, long K) {
 // 1024 x 5504 x 16384 715 -> 447, 1024 x 5504 x 5000 219 -> 150, 2048 x 768 x
 // 8000 100 -> 71, 1024 x 1024 x 4096 30 -> 42, 2752 x 1024 x 2048 36 -> 43.)
 bool pp_wins_dw(long M, long N, long K, int& splits) {
+  static const bool off = overridden({"SJ_GEMM_DW_TILE", "SJ_GEMM_DW_SPLITS", "SJ_GEMM_KW", "SJ_GEMM_KW_SPLITS"});
   splits = 1;
+  if (off || pp_off()) return false;
   const double mn = (double)M * (double)N;
   const long t = tiles(M, N, 256, 128), cu = cus();
   double best = 0;
@@ -2086,6 +2109,36 @@ extern "C" size_t sj_gemm_planes_workspace_bytes(long M, long N, long K) {
     need = b > need ? b : need;
   }
   return need;
+}
+
+// The same rules, in the order the entry points ask them.
+extern "C" int sj_gemm_planes_plan(int op, long M, long N, long K, int* bm, int* bn, int* splits) {
+  SJ_REQUIRE(op >= 0 && op <= 5 && M > 0 && N > 0 && K > 0 && bm && bn && splits, "product plan: op %d", op);
+  *splits = 1;
+  const int epi[5] = {E_STORE, E_STORE, E_GATEUP, E_RESID, E_PLANES};
+  if (op == 1) {
+    *bm = 256;
+    *bn = 128;
+    if (pp_wins_dw(M, N, K, *splits)) return 2;
+    *bm = *bn = 64;
+    if (plan_kw(M, N, K, 1, *splits)) return 1;
+    plan(M, N, K, 1, *bm, *bn, *splits, true);
+    return 0;
+  }
+  if (op < 5 && N % 8 == 0 && pp_wins(epi[op], M, N, K)) {
+    *bm = op == 0 || op == 4 ? 128 : 256;
+    *bn = op == 2 ? 128 : 256;
+    return 2;
+  }
+  if (op == 2 || op == 3) {
+    pick(M, N, *bm, *bn);
+    if (op == 2 && *bm == 128 && *bn == 128) *bn = 64;
+    return 0;
+  }
+  plan(M, N, K, 2, *bm, *bn, *splits, op == 5);
+  if (op == 4) *splits = 1;
+  if (op == 5) plan_tall(M, N, K, *bm, *bn, *splits);
+  return 0;
 }
 
 namespace {

@@ -1940,11 +1940,19 @@ bool pp_wins(int epi, long M, long N, long K) {
 }
 
 // The same for a dW product (both operands in row layout, Y in two planes),
-// with its K slices.  k_gemm_fast's time follows its plan: stages of 64 k at
-// 1.42 us for a 128 x 128 tile (one per CU), 1.05 for 128 x 64 (two) and 0.78
-// for 64 x 64 (three); k_gemm_kw's steps of 128 tokens take 0.8.  (us:
-// 1024 x 5504 x 16384 715 -> 447, 1024 x 5504 x 5000 219 -> 150, 2048 x 768 x
-// 8000 100 -> 71, 1024 x 1024 x 4096 30 -> 42, 2752 x 1024 x 2048 36 -> 43.)
+// with its K slices.  A stage of 32 k takes 0.45 us + 0.55 x the share of the
+// CUs at work, and with few of them no less than its own latency, 0.65 us + 0.17
+// x the share.  The other side follows its plan: stages of 64 k at 1.5 us for a
+// 128 x 128 tile (one per CU), 1.05 for 128 x 64 (two; 0.78 up to about one)
+// and 0.85 for 64 x 64 (three; 0.78, 0.68 and 0.5 up to two, one and a half and
+// one); k_gemm_kw's steps of 128 tokens take 0.8.  Over 865 shapes of 64-6000
+// columns and 512-40000 tokens the products that it takes are up to three times
+// as fast for it, and two are slower, by 3 and 7% (without the few-workgroup
+// terms 61 of 250 took 1.1-1.7 times as long).  us, old -> this: 1024 x 5504 x
+// 16384 655 -> 399, 1024 x 1536 x 16384 181 -> 101, 2752 x 1024 x 16384 219 ->
+// 212, 232 x 3408 x 30458 245 -> 123; not taken: 1024 x 1024 x 4096 29 (42
+// here), 2752 x 1024 x 2048 31 (43), 904 x 312 x 2769 25 (42), 656 x 72 x 25112
+// 54 (85).
 bool pp_wins_dw(long M, long N, long K, int& splits) {
   static const bool off = overridden({"SJ_GEMM_DW_TILE", "SJ_GEMM_DW_SPLITS", "SJ_GEMM_KW", "SJ_GEMM_KW_SPLITS"});
   splits = 1;
@@ -1953,7 +1961,9 @@ bool pp_wins_dw(long M, long N, long K, int& splits) {
   const long t = tiles(M, N, 256, 128), cu = cus();
   double best = 0;
   for (int s = 1; s <= PP_SPLITS && (s == 1 || K / s >= 1024); s++) {
-    const double c = pp_us(t * s, (double)K / PP_K / s, 6.0, 0.45, 0.55) + (s > 1 ? 4.0 + s * mn * 8.0 / 4.5e6 : 0.0);
+    const double few = pp_us(t * s, (double)K / PP_K / s, 6.0, 0.65, 0.17);
+    const double full = pp_us(t * s, (double)K / PP_K / s, 6.0, 0.45, 0.55);
+    const double c = (few > full ? few : full) + (s > 1 ? 4.0 + s * mn * 8.0 / 4.5e6 : 0.0);
     if (s == 1 || c < best) {
       best = c;
       splits = s;
@@ -1965,13 +1975,14 @@ bool pp_wins_dw(long M, long N, long K, int& splits) {
     old = 2.0 + (double)K / 128 / so * 0.8;
   } else {
     plan(M, N, K, 1, bm, bn, so, true);
-    const bool one = bm == 128 && bn == 128;
-    const long slots = one ? cu : bm + bn == 192 ? 2 * cu : 3 * cu;
-    old = 3.0 + (double)((tiles(M, N, bm, bn) * so + slots - 1) / slots) * ((double)K / 64 / so) *
-                    (one ? 1.42 : bm + bn == 192 ? 1.05 : 0.78);
+    const long wgs = tiles(M, N, bm, bn) * so, per = bm + bn == 256 ? 1 : bm + bn == 192 ? 2 : 3;
+    const double stage = per == 1   ? 1.5
+                         : per == 2 ? (10 * wgs <= 11 * cu ? 0.78 : 1.05)
+                                    : (wgs <= cu ? 0.5 : 2 * wgs <= 3 * cu ? 0.68 : wgs <= 2 * cu ? 0.78 : 0.85);
+    old = 3.0 + (double)((wgs + per * cu - 1) / (per * cu)) * ((double)K / 64 / so) * stage;
   }
   if (so > 1) old += 4.0 + so * mn * 8.0 / 4.5e6;
-  return best < 0.92 * old;
+  return best < old;
 }
 // bf16 outputs (and inputs) of the ping-pong epilogues: 16-byte accesses of eight columns
 bool pp_cols_ok(const FParams& p, int nout) {

@@ -53,3 +53,15 @@ def test_sweep_overrides_reach_the_large_products():
     assert plans_under(SJ_GEMM_KW="0")[6][0] == FAST
     assert plans_under(SJ_GEMM_KW_SPLITS="2")[6] == (KW, 64, 64, 2)
     assert all(p[0] != PP for p in plans_under(SJ_GEMM_STAGES="2"))
+
+
+# measured on an MI355X, us: the kernels before k_gemm_pp, k_gemm_pp
+@pytest.mark.parametrize("M,N,K,old,pp", [
+    (112, 88, 2447, 22, 35), (904, 312, 2769, 25, 42), (648, 416, 2912, 26, 45), (120, 80, 7947, 22, 35),
+    (664, 264, 21918, 51, 73), (1912, 80, 38089, 84, 119), (3040, 128, 35146, 92, 114), (104, 5672, 3337, 29, 35),
+    (320, 5600, 7001, 85, 95), (656, 72, 25112, 54, 85), (1024, 1024, 4096, 29, 42), (2752, 1024, 2048, 31, 43),
+    (1024, 5504, 16384, 655, 399), (2752, 1024, 16384, 219, 212), (1024, 1536, 16384, 181, 101),
+    (232, 3408, 30458, 238, 116), (4320, 144, 18282, 134, 80), (2056, 552, 37632, 551, 200), (504, 1440, 11264, 71, 49),
+    (5288, 816, 768, 40, 27), (5936, 4840, 12544, 2056, 1308)])
+def test_dw_products_take_the_faster_kernel(M, N, K, old, pp):
+    assert (plan(DW, M, N, K)[0] == PP) == (pp < old)

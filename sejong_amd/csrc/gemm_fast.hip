@@ -1909,9 +1909,12 @@ double pp_us(long t, double stages, double fixed, double a0, double a1) {
 
 // Whether the ping-pong kernel is the faster one for the epilogue's product of
 // k-contiguous operands.  Both sides are modelled from twelve block shapes of
-// 2048-16384 rows and widths of 384-1024 (us, k_gemm_fast -> k_gemm_pp):
+// 2048-16384 rows and widths of 384-1024, gate|up from 151 of 512-40000 rows
+// and widths of 64-6000 (us, k_gemm_fast -> k_gemm_pp):
 //   gate|up      16384 x 2752 x 1024 278 -> 228, 8000 x 2048 x 768 97 -> 74,
-//                4096 x 1024 x 384 19 -> 24, 6000 x 1376 x 512 46 -> 48
+//                4096 x 1024 x 384 19 -> 24, 6000 x 1376 x 512 46 -> 48; with a
+//                last round of few tiles it loses: 11537 x 864 x 3368 177 ->
+//                190, 12699 x 5720 x 400 272 -> 298 (not taken)
 //   residual     16384 x 1024 x 2752 122 -> 98, 8192 x 1024 x 1024 31 -> 40
 //   dX           8000 x 768 x 4096 141 -> 110, 4096 x 1024 x 3072 58 -> 70
 //   split output 8192 x 1024 x 1024 53 -> 45, 4096 x 1024 x 1024 27 -> 34
@@ -1924,8 +1927,15 @@ bool pp_wins(int epi, long M, long N, long K) {
   const double mn = (double)M * (double)N, st = (double)K / PP_K, fl = 2.0 * mn * (double)K;
   double pp, old;
   if (epi == E_GATEUP) {
-    pp = pp_us(tiles(M, N, 256, 128), st, 18.0, 0.65, 0.0);
+    const long t = tiles(M, N, 256, 128);
+    pp = pp_us(t, st, 18.0, 0.65, 0.0);
     old = 4.0 + 2.0 * fl / 0.75e9 + 6.0 * mn / 4e6;
+    // Past one round a last round of few tiles, and the stores of three
+    // outputs, can take the gain: of 151 drawn shapes none that is left to
+    // this kernel is more than 2% slower for it (without these lines 1.04-1.15
+    // times at five).
+    if (t > cus() && 1.2 + pp_us(t, st, 0.0, 0.56, 0.23) + mn / 0.5e6 > 0.95 * (10.2 + 2.0 * fl / 0.89e9 + mn / 0.69e6))
+      return false;
   } else if (epi == E_RESID) {
     pp = pp_us(tiles(M, N, 256, 256), st, 14.0, 0.55, 0.42);
     old = 4.0 + fl / 0.9e9 + 4.0 * mn / 4e6;

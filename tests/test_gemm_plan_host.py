@@ -65,3 +65,12 @@ def test_sweep_overrides_reach_the_large_products():
     (5288, 816, 768, 40, 27), (5936, 4840, 12544, 2056, 1308)])
 def test_dw_products_take_the_faster_kernel(M, N, K, old, pp):
     assert (plan(DW, M, N, K)[0] == PP) == (pp < old)
+
+
+@pytest.mark.parametrize("M,N,K,old,pp", [
+    (11537, 864, 3368, 177, 190), (12699, 5720, 400, 272, 298), (23308, 456, 3928, 225, 259), (5532, 1816, 3816, 206, 218),
+    (16562, 656, 5832, 322, 335), (4096, 1024, 384, 19, 24), (16384, 2752, 1024, 278, 228), (8000, 2048, 768, 97, 74),
+    (1206, 4784, 3512, 124, 93), (28568, 176, 5952, 196, 144), (4472, 1040, 4184, 146, 114), (15200, 2584, 400, 156, 115),
+    (9079, 848, 720, 44, 34)])
+def test_gate_up_products_take_the_faster_kernel(M, N, K, old, pp):
+    assert (plan(GATE_UP, M, N, K)[0] == PP) == (pp < old)

@@ -1655,9 +1655,10 @@ int splits_for(long M, long N, long K, int bm, int bn);
 //   very long K (>= 8192) with a short output (M <= 512 or N <= 64: the
 //   token-contracted products of the parameter VJP): 64x64 tiles and
 //   floor(4 x CUs / tiles) K slices, clamped to 8..16 and to slices of
-//   >= 512 (cfg5 coefficients 144 x 1536 x 16384: 14 slices, 66 -> 51 us;
-//   144 x 5504 x 16384: 8 slices, 175 -> 158 us; 64x128 tiles lose at every
-//   slice count);
+//   >= 512 (144 x 1536 x 16384: 14 slices, 66 -> 51 us; 144 x 5504 x 16384: 8
+//   slices, 175 -> 158 us; 64x128 tiles lose at every slice count); the
+//   coefficient product then asks plan_tall, which replaces both where taller
+//   tiles are the faster;
 //   dW-shaped products (K >= 2048, at most one 64x64 tile per CU): one K
 //   slice up to K = 4096, else 4, and the largest tile giving min(2 per CU,
 //   slices x the 64x64 tiles) workgroups (cfg5 attention-output dW: 128x64
@@ -1789,36 +1790,48 @@ bool overridden(std::initializer_list<const char*> names) {
 // Tiles of the parameter VJP's coefficient product (C = A Y, both operands
 // hi/lo planes, Y in row layout, few rows of A against long K).  It is bound
 // by the LDS DMA: a 64 x 64 tile stages 2 x (64 + 64) rows for 3 x 64 x 64
-// products and Y once per row tile.  A tile over all the rows (96, 160 or
-// 192) and 64 or 128 columns stages both less often; what a CU then moves was
-// about 55 KB/us with two workgroups resident and 43 with one.  The plan takes
-// the tile and the K slices (at most the general plan's: the workspace holds
-// those) with the least modelled time: rounds of workgroups, each K / slices
-// stages, and the partials' write and read.  144 x 5504 x 16384: 155 (64 x 64)
-// -> 107 us; 64-row tiles stay with the general plan.
+// products and Y once per row tile.  A tile over all the rows (96 to 192) and
+// 64 or 128 columns stages both less often, but a CU with one workgroup
+// resident moves less (KB/us: 64 x 64 66, two resident; one resident 42 with 64
+// columns, 38 with 128, 34 past 128 x 128).  The plan takes the tile and the K
+// slices (at most the general plan's: the workspace holds those; at least half,
+// so that a sum is at most twice as long) with the least modelled time: rounds
+// of workgroups, each K / slices stages, and the partials' write and read.
+// Where one round holds the general plan's workgroups its stages wait less and
+// it stays (55 x 472 x 49920 37 us, 52 here).  us, general -> this:
+// 144 x 5504 x 16384 159 -> 117, 272 x 2048 x 16384 84 -> 65, 122 x 2504 x 64032
+// 287 -> 195; of 280 drawn shapes seven are 3-16% slower (199 x 1920 x 44904
+// 184 -> 204).  Error against 64 bits, 1e-6 relative: 2.801 -> 2.828 at the
+// first (8 -> 5 slices), the same where the slices are.
+// The lines at K and M keep to the parameter VJP's shapes; past them the tiles
+// measured ahead too (235 x 3088 x 7784 0.92 of the general plan's time,
+// 725 x 1104 x 16664 0.82).
 bool plan_tall(long M, long N, long K, int& bm, int& bn, int& splits) {
   static const bool off = overridden({"SJ_GEMM_TILE", "SJ_GEMM_SPLITS", "SJ_GEMM_LK_TILE", "SJ_GEMM_LK_SPLITS"});
-  if (off || K < 8192 || M > 512) return false;
   const long cu = cus();
+  if (off || K < 8192 || M > 512 || tiles(M, N, 64, 64) * splits <= 2 * cu) return false;
   double best = 0;
   int bs = 1, bbm = 0, bbn = 0;
-  for (int cn : {64, 128})
-    for (int cm : {64, 96, 128, 160, 192}) {
-      const long t = tiles(M, N, cm, cn);
-      const double stage = 0.25 * (cm + cn);  // KB: 2 (cm + cn) rows of 128 bytes
-      const int occ = 4 * stage <= 160 ? 2 : 1;
-      const double per = (double)occ * stage / (occ == 2 ? 55.0 : 43.0);  // us a stage
-      for (int s = 1; s <= splits; s++) {
-        const double c = (double)((t * s + cu * occ - 1) / (cu * occ)) * ((double)K / 64 / s) * per +
-                         (s > 1 ? s * (double)M * (double)N * 8.0 / 4.5e6 : 0.0);
-        if (best == 0 || c < best) {
-          best = c;
-          bs = s;
-          bbm = cm;
-          bbn = cn;
-        }
+  // 96 x 128, 128 x 64 and 192 x 64 are at no shape the least
+  constexpr int cand[6][2] = {{64, 64}, {96, 64}, {160, 64}, {128, 128}, {160, 128}, {192, 128}};
+  for (const auto& c : cand) {
+    const int cm = c[0], cn = c[1];
+    const long t = tiles(M, N, cm, cn);
+    const double stage = 0.25 * (cm + cn);  // KB: 2 (cm + cn) rows of 128 bytes
+    const int occ = 4 * stage <= 160 ? 2 : 1;
+    const double rate = occ == 2 ? (cm == 64 ? 66.0 : 58.0) : stage > 64 ? 34.0 : cn == 64 ? 42.0 : 38.0;
+    const double per = (double)occ * stage / rate;  // us a stage
+    for (int s = (splits + 1) / 2; s <= splits; s++) {
+      const double us = (double)((t * s + cu * occ - 1) / (cu * occ)) * ((double)K / 64 / s) * per +
+                        (s > 1 ? s * (double)M * (double)N * 8.0 / 4.5e6 : 0.0);
+      if (best == 0 || us < best) {
+        best = us;
+        bs = s;
+        bbm = cm;
+        bbn = cn;
       }
     }
+  }
   if (bbm == 64) return false;
   bm = bbm;
   bn = bbn;
@@ -1828,13 +1841,7 @@ bool plan_tall(long M, long N, long K, int& bm, int& bn, int& splits) {
 
 template <int EPI>
 int launch_tall(hipStream_t s, const FParams& p, int bm, int bn, int splits) {
-  if (bn == 64) {
-    if (bm == 96) return launch<96, 64, 2, 2, EPI, 2>(s, p, splits);
-    if (bm == 128) return launch<128, 64, 2, 2, EPI, 2>(s, p, splits);
-    if (bm == 160) return launch<160, 64, 2, 2, EPI, 2>(s, p, splits);
-    return launch<192, 64, 2, 2, EPI, 2>(s, p, splits);
-  }
-  if (bm == 96) return launch<96, 128, 2, 2, EPI, 2>(s, p, splits);
+  if (bn == 64) return bm == 96 ? launch<96, 64, 2, 2, EPI, 2>(s, p, splits) : launch<160, 64, 2, 2, EPI, 2>(s, p, splits);
   if (bm == 128) return launch<128, 128, 2, 2, EPI, 2>(s, p, splits);
   if (bm == 160) return launch<160, 128, 2, 2, EPI, 2>(s, p, splits);
   return launch<192, 128, 2, 2, EPI, 2>(s, p, splits);
@@ -2036,8 +2043,6 @@ template <int EPI>
 int set_attrs_tall() {
   int s = set_attr<96, 64, 2, 2, EPI, 2>();
   if (!s) s = set_attr<160, 64, 2, 2, EPI, 2>();
-  if (!s) s = set_attr<192, 64, 2, 2, EPI, 2>();
-  if (!s) s = set_attr<96, 128, 2, 2, EPI, 2>();
   if (!s) s = set_attr<128, 128, 2, 2, EPI, 2>();
   if (!s) s = set_attr<160, 128, 2, 2, EPI, 2>();
   if (!s) s = set_attr<192, 128, 2, 2, EPI, 2>();

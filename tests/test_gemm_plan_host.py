@@ -74,3 +74,16 @@ def test_dw_products_take_the_faster_kernel(M, N, K, old, pp):
     (9079, 848, 720, 44, 34)])
 def test_gate_up_products_take_the_faster_kernel(M, N, K, old, pp):
     assert (plan(GATE_UP, M, N, K)[0] == PP) == (pp < old)
+
+
+@pytest.mark.parametrize("M,N,K,general,tall", [
+    (55, 472, 49920, 37, 52), (176, 256, 65536, 46, 66), (48, 1024, 16384, 19, 24), (112, 512, 8192, 15, 18),
+    (96, 768, 12000, 19, 22), (115, 104, 68408, 48, 78), (360, 320, 35624, 40, 48), (432, 576, 28104, 63, 71),
+    (386, 768, 46400, 108, 127), (144, 5504, 16384, 159, 117), (144, 2752, 16384, 76, 67), (272, 2048, 16384, 84, 65),
+    (144, 1536, 16384, 42, 39), (154, 4784, 14832, 157, 101), (122, 2504, 64032, 287, 195), (144, 1024, 16384, 35, 30)])
+def test_coefficient_products_take_the_faster_tile(M, N, K, general, tall):
+    _, bm, bn, splits = plan(COEFFICIENTS, M, N, K)
+    assert ((bm, bn) != (64, 64)) == (tall < general)
+    # no slice more than twice the general plan's: its sums' error grows with the length
+    t = -(-M // 64) * -(-N // 64)
+    assert 2 * splits >= min(max(4 * 256 // t, 8), 16)

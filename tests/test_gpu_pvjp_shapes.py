@@ -1,6 +1,6 @@
 """The parameter VJP's kernels at the edges of their ranges: ranks 1, 16, 17,
 32, 33 and 64, ragged rows, more than 64 selected blocks (the serial draws),
-and the coefficient product's row tiles (64, 96, 128, 160, 192 rows)."""
+and the coefficient product's tiles (64 x 64, and each taller one)."""
 import ctypes
 
 import numpy as np
@@ -8,6 +8,7 @@ import pytest
 
 from oracle import oracle as O
 from oracle import pvjp as P
+from tests.test_gemm_plan_host import COEFFICIENTS, plan
 from tests.gpu_util import best_us, dev, empty, rel, rnd, sync, zeros
 
 pytestmark = pytest.mark.gpu
@@ -97,11 +98,15 @@ def test_basis_value_out_of_range_stays_in_its_row(N, R, bad):
     assert np.isfinite(np.delete(q.host().reshape(n, R), 41, axis=0)).all()
 
 
-@pytest.mark.parametrize("rows,b,n", [(48, 200, 8192), (80, 136, 8200), (112, 64, 8192), (144, 264, 8256),
-                                      (176, 72, 16384), (272, 320, 8192), (145, 8, 9000)])
-def test_coefficient_tiles(N, rows, b, n):
+@pytest.mark.parametrize("rows,b,n,tile", [
+    (48, 200, 8192, (64, 64)), (80, 136, 8200, (64, 64)), (112, 64, 8192, (64, 64)), (144, 264, 8256, (64, 64)),
+    (176, 72, 16384, (64, 64)), (272, 320, 8192, (64, 64)), (145, 8, 9000, (64, 64)),
+    (66, 1504, 8456, (96, 64)), (129, 976, 8288, (160, 64)), (100, 2056, 8208, (128, 128)), (129, 3344, 8648, (160, 128)),
+    (162, 3296, 8312, (192, 128))])
+def test_coefficient_tiles(N, rows, b, n, tile):
     """E dY with both operands as hi/lo planes, dY in row layout: against FP64
     (three bf16 products of four: 2^-16 per term, random signs)."""
+    assert plan(COEFFICIENTS, rows, b, n)[1:3] == tile
     rng = np.random.default_rng(rows + b)
     split = lambda x: (O.round_to(x, "bf16"), O.round_to(x - O.round_to(x, "bf16"), "bf16"))
     e = rng.normal(0, 1, (rows, n)).astype(np.float32).astype(np.float64)

@@ -263,8 +263,18 @@ __global__ __launch_bounds__(NT) void k_gemm(GemmParams p) {
     kend = kbeg + p.kchunk < p.K ? kbeg + p.kchunk : p.K;
   }
 
-  // k-steps in flight: as many as the registers of a tile leave room for
-  constexpr int PD = BM * BN > 64 * 64 ? 2 : DUAL ? 3 : 4;
+  // k-steps in flight: as many as the registers of a tile leave room for.  Two
+  // bf16 operands move half the bytes a step and their large tiles fill the
+  // chip with workgroups; there the registers of a second step cost more (a
+  // wave per SIMD) than it hides, and with both operands strided along k
+  // (kinds 1, 1) at every tile: 8192 x 4096 x 512 A^T B 70 us with one, 86 with
+  // two; 16384 x 1024 x 1024 A B^T 57 and 68; 1024 x 1024 x 4096 A^T B 87 and 111
+  // with four.
+  constexpr bool BF2 = !AF && !BF;
+  constexpr int PD = BF2 && ((AK == 1 && BKND == 1) || BM * BN == 128 * 128 || (BM * BN == 128 * 64 && BKND == 1)) ? 1
+                     : BM * BN > 64 * 64                                                                          ? 2
+                     : DUAL                                                                                       ? 3
+                                                                                                                  : 4;
   Loader<AK, BM> la[PD];
   Loader<BKND, BN> lb0[PD];
   Loader<BKND, BN> lb1[DUAL ? PD : 1];

@@ -55,3 +55,13 @@ def test_no_kernel_spills_its_work(kernels):
     spilled = {n: k[".private_segment_fixed_size"] for n, k in kernels.items()
                if k[".private_segment_fixed_size"] > 64}
     assert not spilled
+
+
+@pytest.mark.parametrize("bm,bn,ak,bk,vgprs", [(128, 128, 0, 0, 128), (128, 128, 1, 1, 168), (128, 64, 1, 1, 128),
+                                               (64, 128, 1, 1, 128)])
+def test_bf16_products_keep_their_waves(kernels, bm, bn, ak, bk, vgprs):
+    """sj_gemm's large bf16 tiles run four (three at 128 x 128 A^T B) waves per
+    SIMD; one fewer, from a second k-step in registers, took up to 1.25x."""
+    tag = f"k_gemmILi{bm}ELi{bn}ELi{ak}ELi{bk}ELi0E"
+    found = [k[".vgpr_count"] for n, k in kernels.items() if tag in n]
+    assert found and max(found) <= vgprs

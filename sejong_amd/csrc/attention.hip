@@ -950,15 +950,15 @@ struct RowArgs {
 };
 
 // The row kernels (fp32, and bf16 shapes outside the MFMA layout): any even
-// head_dim up to 128, any window.  Their first form gave one wave a row and
-// walked its keys one at a time (a dot product over the lanes, a six-step
-// wave sum, the exponential, the accumulate): a serial chain of about 60 ns
-// a key, at most half the lanes in use below head_dim 64.  Here a workgroup
-// stages 64 streamed rows (keys, or queries for dK | dV) in LDS and each wave
+// head_dim up to 128, any window.  The plain form (k_attn_*_walk below, kept for
+// short walks) gives one wave a row and walks its keys one at a time (a dot
+// product over the lanes, a six-step wave sum, the exponential, the
+// accumulate): a serial chain of about 60 ns a key, at most half the lanes in
+// use below head_dim 64.  Here a workgroup stages 64 streamed rows (keys, or queries for dK | dV) in LDS and each wave
 // takes R fixed rows against them in two phases.  First lane j forms streamed
 // row j's whole dot product, and the softmax terms of 64 rows at once; then
 // the lanes turn to the columns (64 / C rows of C columns at a time) and add
-// the weighted rows one after another.  Every sum keeps the first form's
+// the weighted rows one after another.  Every sum keeps the plain form's
 // order (the dot product's pairwise tree over the columns, keys in order, the
 // running maximum after each key as a prefix maximum), so the results have
 // its bits, and a row's bits depend on its position alone: the cached forward
@@ -1302,6 +1302,152 @@ __global__ __launch_bounds__(256) void k_attn_bwd_rows(RowArgs a) {
   }
 }
 
+// The same rows, one wave each, keys (or queries) one at a time: a dot product
+// over the lanes, a wave sum, the exponential, the accumulate, about 60 ns of
+// serial latency a key.  It serves the short walks (a window or sequence of a
+// few rows), where staging 64 rows costs more than it saves; the two forms
+// take the same operations in the same order.
+template <bool CACHED>
+__global__ __launch_bounds__(256) void k_attn_fwd_walk(RowArgs a) {
+  const int lane = threadIdx.x & 63;
+  const long row = blockIdx.x * 4L + (threadIdx.x >> 6);  // (b*T + pos)*HQ + h
+  if (row >= a.B * a.T * a.HQ) return;
+  const long h = row % a.HQ, bt = row / a.HQ, pos = CACHED ? a.offset + bt : bt % a.T, b = CACHED ? 0 : bt / a.T;
+  const long kvh = h / (a.HQ / a.HK);
+  const float scale = 1.f / sqrtf((float)a.D);
+  float q[2], acc[2] = {0.f, 0.f};
+  for (int i = 0; i < 2; i++) {
+    long d = lane + 64 * i;
+    q[i] = d < a.D ? load_as_f32(a.q, a.dt, bt * a.ldq + h * a.D + d) : 0.f;
+  }
+  float m = -INFINITY, l = 0.f;
+  long first = a.window > 0 ? (pos + 1 - a.window > 0 ? pos + 1 - a.window : 0) : 0;
+  for (long p = first; p <= pos; p++) {
+    long kr = (b * a.T + p);
+    float s = 0.f;
+    for (int i = 0; i < 2; i++) {
+      long d = lane + 64 * i;
+      if (d < a.D) s += q[i] * load_as_f32(a.k, a.dt, kr * a.ldk + kvh * a.D + d);
+    }
+    s = wave_sum(s) * scale;
+    float mn = fmaxf(m, s);
+    float al = expf(m - mn), pr = expf(s - mn);
+    for (int i = 0; i < 2; i++) {
+      long d = lane + 64 * i;
+      float vv = d < a.D ? load_as_f32(a.v, a.dt, kr * a.ldv + kvh * a.D + d) : 0.f;
+      acc[i] = acc[i] * al + pr * vv;
+    }
+    l = l * al + pr;
+    m = mn;
+  }
+  for (int i = 0; i < 2; i++) {
+    long d = lane + 64 * i;
+    if (d < a.D) store_from_f32(a.out, a.dt, bt * a.ldo + h * a.D + d, acc[i] / l);
+  }
+  if (!CACHED && lane == 0) a.lse[row] = m + logf(l);
+}
+
+__device__ __forceinline__ void inv_rope_store(float* dst, const float* rope, long pos, long D, int lane, float x0,
+                                               float x1) {
+  // lanes hold consecutive columns; pair partner is lane ^ 1 (D even)
+  float y0 = __shfl_xor(x0, 1, 64), y1 = __shfl_xor(x1, 1, 64);
+  float xs[2] = {x0, x1}, ys[2] = {y0, y1};
+  for (int i = 0; i < 2; i++) {
+    long d = lane + 64 * i;
+    if (d < D) {
+      float x = xs[i];
+      if (rope) {
+        float2 cs = *(const float2*)(rope + 2 * (pos * (D / 2) + (d >> 1)));
+        x = (d & 1) ? (x * cs.x - ys[i] * cs.y) : (x * cs.x + ys[i] * cs.y);
+      }
+      dst[d] = x;
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void k_attn_dq_walk(RowArgs a) {
+  const int lane = threadIdx.x & 63;
+  const long row = blockIdx.x * 4L + (threadIdx.x >> 6);
+  if (row >= a.B * a.T * a.HQ) return;
+  const long h = row % a.HQ, bt = row / a.HQ, pos = bt % a.T, b = bt / a.T;
+  const long kvh = h / (a.HQ / a.HK);
+  const float scale = 1.f / sqrtf((float)a.D);
+  float q[2], dy[2], acc[2] = {0.f, 0.f};
+  float dl = 0.f;
+  for (int i = 0; i < 2; i++) {
+    long d = lane + 64 * i;
+    q[i] = d < a.D ? load_as_f32(a.q, a.dt, bt * a.ldq + h * a.D + d) : 0.f;
+    dy[i] = d < a.D ? a.dout[bt * a.lddo + h * a.D + d] : 0.f;
+    float ov = d < a.D ? load_as_f32(a.o, a.dt, bt * a.ldo + h * a.D + d) : 0.f;
+    dl += dy[i] * ov;
+  }
+  dl = wave_sum(dl);
+  if (lane == 0) a.delta[row] = dl;
+  const float lse = a.lse[row];
+  long first = a.window > 0 ? (pos + 1 - a.window > 0 ? pos + 1 - a.window : 0) : 0;
+  for (long p = first; p <= pos; p++) {
+    long kr = b * a.T + p;
+    float s = 0.f, dp = 0.f, kv[2];
+    for (int i = 0; i < 2; i++) {
+      long d = lane + 64 * i;
+      kv[i] = d < a.D ? load_as_f32(a.k, a.dt, kr * a.ldk + kvh * a.D + d) : 0.f;
+      float vv = d < a.D ? load_as_f32(a.v, a.dt, kr * a.ldv + kvh * a.D + d) : 0.f;
+      s += q[i] * kv[i];
+      dp += dy[i] * vv;
+    }
+    s = wave_sum(s);
+    dp = wave_sum(dp);
+    float pr = expf(s * scale - lse);
+    float ds = pr * (dp - dl) * scale;
+    for (int i = 0; i < 2; i++) acc[i] += ds * kv[i];
+  }
+  inv_rope_store(a.dq + bt * a.lddq + h * a.D, a.rope, pos, a.D, lane, acc[0], acc[1]);
+}
+
+__global__ __launch_bounds__(256) void k_attn_dkv_walk(RowArgs a) {
+  const int lane = threadIdx.x & 63;
+  const long row = blockIdx.x * 4L + (threadIdx.x >> 6);  // (b*T + pos)*HK + kvh
+  if (row >= a.B * a.T * a.HK) return;
+  const long kvh = row % a.HK, bt = row / a.HK, pos = bt % a.T, b = bt / a.T;
+  const long group = a.HQ / a.HK;
+  const float scale = 1.f / sqrtf((float)a.D);
+  float k[2], v[2], ak[2] = {0.f, 0.f}, av[2] = {0.f, 0.f};
+  for (int i = 0; i < 2; i++) {
+    long d = lane + 64 * i;
+    k[i] = d < a.D ? load_as_f32(a.k, a.dt, bt * a.ldk + kvh * a.D + d) : 0.f;
+    v[i] = d < a.D ? load_as_f32(a.v, a.dt, bt * a.ldv + kvh * a.D + d) : 0.f;
+  }
+  long end = a.window > 0 ? (pos + a.window < a.T ? pos + a.window : a.T) : a.T;
+  for (long gi = 0; gi < group; gi++) {
+    long h = kvh * group + gi;
+    for (long qp = pos; qp < end; qp++) {
+      long qr = (b * a.T + qp);
+      float s = 0.f, dp = 0.f, qv[2], dy[2];
+      for (int i = 0; i < 2; i++) {
+        long d = lane + 64 * i;
+        qv[i] = d < a.D ? load_as_f32(a.q, a.dt, qr * a.ldq + h * a.D + d) : 0.f;
+        dy[i] = d < a.D ? a.dout[qr * a.lddo + h * a.D + d] : 0.f;
+        s += qv[i] * k[i];
+        dp += dy[i] * v[i];
+      }
+      s = wave_sum(s);
+      dp = wave_sum(dp);
+      long qrow = qr * a.HQ + h;
+      float pr = expf(s * scale - a.lse[qrow]);
+      float ds = pr * (dp - a.delta[qrow]) * scale;
+      for (int i = 0; i < 2; i++) {
+        ak[i] += ds * qv[i];
+        av[i] += pr * dy[i];
+      }
+    }
+  }
+  inv_rope_store(a.dk + bt * a.lddk + kvh * a.D, a.rope, pos, a.D, lane, ak[0], ak[1]);
+  for (int i = 0; i < 2; i++) {
+    long d = lane + 64 * i;
+    if (d < a.D) a.dv[bt * a.lddv + kvh * a.D + d] = av[i];
+  }
+}
+
 // Rows per wave: 4 once that gives two workgroups per CU (a staged row then
 // serves 16 fixed ones); below, as many as fill the lanes with columns
 // (shorter chains, more workgroups).
@@ -1335,8 +1481,31 @@ void rt_pick(long D, long rows_heads, F f) {
   SJ_RT(128, 4);
 #undef SJ_RT
 }
+// Whether the walk of a row (its window, or its sequence's length) is short
+// enough for the one-key-at-a-time kernels.  Time of the staged kernels over
+// theirs, forward / backward, fp32, 8 x 1024 tokens (4 x 1024 at head_dim 96 and
+// 128; at 2 x 512 and below the launch hides most of it):
+//   window        1          4          8          12         16         24
+//   head_dim 16   0.98/0.96  0.71/0.65  0.44/0.41
+//   32            1.40/1.79  0.87/1.06  0.60/0.63
+//   64            2.10/2.99  1.30/1.95  0.88/1.24  0.68/0.88
+//   96            7.19/9.64  4.31/5.25  2.89/3.19  2.19/2.26  1.83/1.77  1.42/1.25
+//   128           5.53/6.02  3.02/3.40  2.00/2.14  1.48/1.62  1.20/1.34  0.89/1.02
+// Sequences of at most 4 tokens leave most of a staged block's 16 rows empty
+// (1024 of 4, head_dim 16: 1.54/1.71).  Above head_dim 64 with one row a wave
+// (few rows) the line is at 12 (256 tokens, head_dim 128: 0.92/1.14).
+bool short_walk(const RowArgs& a, long heads) {
+  const long len = a.offset + a.T, span = a.window > 0 && a.window < len ? a.window : len;
+  const int C = rt_cols(a.D);
+  return span <= (C <= 16 ? (len <= 4 ? 4 : 2) : C == 32 ? 4 : C == 64 ? 8 : rt_rows(a.D, a.B * a.T * heads) == 4 ? 24 : 12);
+}
+
 template <template <int, int> class K>
-void launch_rows(hipStream_t s, const RowArgs& a, long heads) {
+void launch_rows(hipStream_t s, const RowArgs& a, long heads, rt_kernel walk) {
+  if (short_walk(a, heads)) {
+    hipLaunchKernelGGL(walk, dim3((unsigned)((a.B * a.T * heads + 3) / 4)), dim3(256), 0, s, a);
+    return;
+  }
   rt_pick<K>(a.D, a.B * a.T * heads, [&](rt_kernel k, int R, size_t lds) {
     const long grid = (a.T + 4 * R - 1) / (4 * R) * heads * a.B;
     hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(256), lds, s, a);
@@ -1403,7 +1572,7 @@ extern "C" int sj_attention_fwd(void* stream, const void* q, long ldq, const voi
     a.out = o; a.lse = lse; a.dt = dtype; a.B = batch; a.T = t; a.HQ = hq; a.HK = hk; a.D = head_dim;
     a.window = window;
     if (int st = rows_prepare()) return st;
-    launch_rows<RtFwd>(s, a, hq);
+    launch_rows<RtFwd>(s, a, hq, k_attn_fwd_walk<false>);
   }
   SJ_LAUNCH_CHECK("hierarchy_attention");
   return SJ_OK;
@@ -1430,7 +1599,7 @@ extern "C" int sj_attention_fwd_cached(void* stream, const void* q, long ldq, co
   a.out = o; a.dt = dtype; a.B = 1; a.T = tq; a.HQ = hq; a.HK = hk; a.D = head_dim;
   a.window = window; a.offset = offset;
   if (int st = rows_prepare()) return st;
-  launch_rows<RtCached>(s, a, hq);
+  launch_rows<RtCached>(s, a, hq, k_attn_fwd_walk<true>);
   SJ_LAUNCH_CHECK("hierarchy_attention (cached)");
   return SJ_OK;
 }
@@ -1468,8 +1637,8 @@ extern "C" int sj_attention_bwd(void* stream, const void* q, long ldq, const voi
     a.dt = dtype; a.B = batch; a.T = t; a.HQ = hq; a.HK = hk; a.D = head_dim; a.window = window;
     a.rope = rope_table;
     if (int st = rows_prepare()) return st;
-    launch_rows<RtDq>(s, a, hq);
-    launch_rows<RtDkv>(s, a, hk);
+    launch_rows<RtDq>(s, a, hq, k_attn_dq_walk);
+    launch_rows<RtDkv>(s, a, hk, k_attn_dkv_walk);
   }
   SJ_LAUNCH_CHECK("hierarchy_attention_backward");
   return SJ_OK;

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
-from tests.gpu_util import assert_stored_close, dev, empty, rel, rnd, sync
+from tests.gpu_util import assert_stored_close, best_us, dev, empty, rel, rnd, sync
 
 pytestmark = pytest.mark.gpu
 DT = {"f32": 0, "bf16": 4}
@@ -29,6 +29,13 @@ CASES = [
     (3, 131, 2, 1, 64, "bf16", 65, 8),   # bf16, ragged T, window
     (4, 520, 4, 2, 24, "f32", 200, 0),   # 16 rows per workgroup
     (2, 1100, 4, 4, 72, "bf16", 0, 0),   # 16 rows per workgroup, bf16, two column halves
+    (4, 519, 8, 4, 64, "f32", 0, 0),     # 16 rows per workgroup in all three kernels at one 64-column group
+    (5, 450, 4, 4, 48, "f32", 77, 4),    # the same, columns not a power of two, a window
+    # the short walks (one key at a time) at their lines, and one past them
+    (2, 70, 2, 1, 16, "f32", 2, 0), (2, 70, 2, 1, 16, "f32", 3, 0), (3, 4, 2, 1, 10, "bf16", 0, 0),
+    (2, 70, 4, 2, 32, "f32", 4, 1), (2, 70, 4, 2, 32, "bf16", 5, 0), (7, 8, 3, 1, 64, "f32", 0, 0),
+    (2, 70, 2, 2, 64, "bf16", 9, 8), (2, 70, 2, 1, 128, "f32", 12, 0), (2, 70, 2, 2, 100, "f32", 13, 0),
+    (4, 1030, 4, 2, 96, "f32", 24, 0), (4, 1030, 4, 2, 96, "f32", 25, 0),
 ]
 
 
@@ -69,6 +76,42 @@ def test_row_kernels_against_oracle(api, B, T, HQ, HK, Dh, dt, window, pad):
     for name, got, ref in (("delta", De, delta), ("dq", dQ, dq), ("dk", dK, dk), ("dv", dV, dv)):
         e = np.linalg.norm(got.host() - np.asarray(ref, np.float64).ravel())
         assert e < 1e-4 * np.linalg.norm(ref) + slack, (name, e)
+
+
+def test_cached_rows_of_both_row_counts_have_the_same_bits(api):
+    """One 64-column group: the full forward takes 16 rows per workgroup, the
+    few cached rows 4; and a window short enough for the walk kernels against
+    the same rows of a cache whose length alone differs."""
+    T, HQ, HK, Dh = 2112, 4, 2, 64
+    d, J = HQ * Dh, HK * Dh
+    rng = np.random.default_rng(64)
+    Q, K, V = (dev(rnd((T, n), "f32", rng)) for n in (d, J, J))
+    for window in (0, 8, 9):
+        O1, LSE, O2 = empty(T * d), empty(T * HQ), empty(5 * d)
+        api.sj_attention_fwd(None, Q.p, d, K.p, J, V.p, J, O1.p, d, LSE.p, 0, 1, T, HQ, HK, Dh, window)
+        for L in (T - 5, 0, 3):
+            api.sj_attention_fwd_cached(None, Q.at(L * d), d, K.p, V.p, J, T, 0, 5, L, HQ, HK, Dh, window, O2.p, d)
+            sync()
+            np.testing.assert_array_equal(O2.host().reshape(5, d), O1.host().reshape(T, d)[L:L + 5])
+
+
+def test_short_windows_cost_less_than_long_ones(api):
+    """A window of 2 walks its few keys: no staged tile of 64 (4 x 1024 tokens,
+    head_dim 128: staged, 2 and 64 took the same time and 4.5 times as long)."""
+    B, T, H, Dh = 4, 1024, 4, 128
+    n = B * T * H * Dh
+    Q, K, V, DO, O1 = (empty(n) for _ in range(5))
+    L, dQ, dK, dV, De = empty(B * T * H), empty(n), empty(n), empty(n), empty(B * T * H)
+    for b in (Q, K, V, DO):
+        api.sj_fill(None, b.p, 0, n, 0.25)
+
+    def us(window):
+        def call():
+            api.sj_attention_fwd(None, Q.p, H * Dh, K.p, H * Dh, V.p, H * Dh, O1.p, H * Dh, L.p, 0, B, T, H, H, Dh, window)
+            api.sj_attention_bwd(None, Q.p, H * Dh, K.p, H * Dh, V.p, H * Dh, O1.p, H * Dh, L.p, DO.p, H * Dh, dQ.p, H * Dh,
+                                 dK.p, H * Dh, dV.p, H * Dh, De.p, 0, B, T, H, H, Dh, window, None)
+        return best_us(call)
+    assert us(2) < 0.5 * us(64)
 
 
 @pytest.mark.parametrize("L,window", [(2111, 0), (2107, 100), (2047, 64), (0, 0)])

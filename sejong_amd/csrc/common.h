@@ -245,11 +245,16 @@ GradSq& grad_sq();
 int fail(int status, const char* fmt, ...);
 int hip_check(hipError_t e, const char* what);
 // f's status (SJ_OK or a failure), run once on each device: the kernel
-// attributes f sets belong to the current device
+// attributes f sets belong to the current device (asking for it costs about
+// 90 ns a call, so a process that sees one device does not)
 template <class F>
 int once_per_device(sj::OncePerDevice& once, F f) {
+  static const int devices = [] {
+    int n = 0;
+    return hipGetDeviceCount(&n) == hipSuccess ? n : 0;
+  }();
   int device = 0;
-  const hipError_t e = hipGetDevice(&device);
+  const hipError_t e = devices == 1 ? hipSuccess : hipGetDevice(&device);
   return e == hipSuccess ? once(device, f) : hip_check(e, "current device");
 }
 // sj_rmsnorm_bwd_p with the dw reduce left to rmsnorm_reduce_multi (partial:

@@ -1100,9 +1100,10 @@ __global__ __launch_bounds__(NT) void k_gemm_kw(FParams p) {
 // next tile's first three stages before it stores the current one: with a
 // workgroup per tile the fill and the stores of 16384 x 2752 x 1024 took as
 // long as its products.  The sums run over k in the same order (per 32 k: hi,
-// then the other plane), so results equal k_gemm_fast's bit for bit (Delta
-// sums its head's columns in another order).  At 16384 x 1024 x 5504, two
-// planes: 420 -> 309 us, 1.2 PFLOP/s, matrix cores 61% busy (27-40% before).
+// then the other plane), so results equal k_gemm_fast's bit for bit where the
+// K slices are the same (dW takes its own: 1e-6 apart; Delta sums its head's
+// columns in another order).  At 16384 x 1024 x 5504, two planes: 420 -> 309 us,
+// 1.2 PFLOP/s, matrix cores busy 48% of the time at 2.4 GHz (35% before).
 constexpr int PP_T = 512, PP_K = 32, PP_STAGE = 512 * PP_K;  // threads, k per stage, elements per stage
 constexpr size_t PP_LDS = (size_t)4 * PP_STAGE * 2;
 

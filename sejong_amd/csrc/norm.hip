@@ -73,7 +73,8 @@ __global__ __launch_bounds__(NT) void k_rms_fwd(const void* __restrict__ x, cons
 }
 
 // A wave's four rows are loaded RB at a time (all four up to d 512; the
-// registers of wider rows hold two or one).
+// registers of wider rows hold two or one).  dx takes the same operations as
+// row by row, contracted otherwise: 5e-8 apart.
 template <int XD, int WD, int NP>
 __global__ __launch_bounds__(NT) void k_rms_bwd(const void* __restrict__ x, const void* __restrict__ w,
                                                 const float* __restrict__ dy, const float* __restrict__ dx_acc,

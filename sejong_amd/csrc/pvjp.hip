@@ -172,8 +172,8 @@ constexpr int GBLK = 256;   // workgroups at most (Gram partials)
 // and the row work; four threads share a row's products, its values coming
 // from LDS, and Q leaves in whole lines.  (A thread per row with a uniform
 // branch per rank and product took 28 us a pass at 16384 x 16, and the Gram
-// of half the workgroups 19 us; the basis of 16384 rows, rank 16, now
-// 48 us from 173, sums and factorisations included.)
+// of half the workgroups 19 us; the basis of 16384 rows, rank 16, back to back
+// 168 -> 36 us, rank 32 477 -> 82, sums and factorisations included.)
 template <int RB, int MODE>
 __global__ __launch_bounds__(256) void k_basis_rows(const void* __restrict__ y, int ydt, long ldy,
                                                     const int32_t* __restrict__ cols, float* __restrict__ q, long n,

@@ -110,22 +110,25 @@ def rel(a, b):
     return np.linalg.norm(a - b) / (n if n > 0 else 1.0)
 
 
-def best_us(call, passes=20, rounds=5):
-    """The shortest mean time of `passes` calls on the default stream, in us."""
-    api, times, ms = _api(), [], ctypes.c_float()
+def best_us(*calls, passes=20, rounds=8):
+    """The shortest mean time of `passes` runs of each call on the default
+    stream, in us; the calls take turns, so that they meet the same clocks."""
+    api, ms = _api(), ctypes.c_float()
+    best = [float("inf")] * len(calls)
     e0, e1 = ctypes.c_void_p(), ctypes.c_void_p()
     api.sj_event_create(ctypes.byref(e0)); api.sj_event_create(ctypes.byref(e1))
-    call()
-    for _ in range(rounds):
-        api.sj_event_record(e0, None)
-        for _ in range(passes):
-            call()
-        api.sj_event_record(e1, None)
-        sync()
-        api.sj_event_elapsed(e0, e1, ctypes.byref(ms))
-        times.append(ms.value * 1000 / passes)
+    for r in range(rounds + 1):
+        for i, call in enumerate(calls):
+            api.sj_event_record(e0, None)
+            for _ in range(passes if r else 1):  # first a warm-up
+                call()
+            api.sj_event_record(e1, None)
+            sync()
+            api.sj_event_elapsed(e0, e1, ctypes.byref(ms))
+            if r:
+                best[i] = min(best[i], ms.value * 1000 / passes)
     api.sj_event_destroy(e0); api.sj_event_destroy(e1)
-    return min(times)
+    return best
 
 
 def release_all():

@@ -105,13 +105,12 @@ def test_short_windows_cost_less_than_long_ones(api):
     for b in (Q, K, V, DO):
         api.sj_fill(None, b.p, 0, n, 0.25)
 
-    def us(window):
-        def call():
-            api.sj_attention_fwd(None, Q.p, H * Dh, K.p, H * Dh, V.p, H * Dh, O1.p, H * Dh, L.p, 0, B, T, H, H, Dh, window)
-            api.sj_attention_bwd(None, Q.p, H * Dh, K.p, H * Dh, V.p, H * Dh, O1.p, H * Dh, L.p, DO.p, H * Dh, dQ.p, H * Dh,
-                                 dK.p, H * Dh, dV.p, H * Dh, De.p, 0, B, T, H, H, Dh, window, None)
-        return best_us(call)
-    assert us(2) < 0.5 * us(64)
+    def both(window):
+        api.sj_attention_fwd(None, Q.p, H * Dh, K.p, H * Dh, V.p, H * Dh, O1.p, H * Dh, L.p, 0, B, T, H, H, Dh, window)
+        api.sj_attention_bwd(None, Q.p, H * Dh, K.p, H * Dh, V.p, H * Dh, O1.p, H * Dh, L.p, DO.p, H * Dh, dQ.p, H * Dh,
+                             dK.p, H * Dh, dV.p, H * Dh, De.p, 0, B, T, H, H, Dh, window, None)
+    short, long = best_us(lambda: both(2), lambda: both(64))
+    assert short < 0.5 * long, (short, long)
 
 
 @pytest.mark.parametrize("L,window", [(2111, 0), (2107, 100), (2047, 64), (0, 0)])

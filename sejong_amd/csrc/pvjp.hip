@@ -512,9 +512,10 @@ __device__ __forceinline__ bool al16(const void* p) { return ((uintptr_t)p & 15)
 // bound by latency): the weights are requested first and travel under the
 // gradient's work, 211 VGPRs.  2 (tables past FSMALL tiles, bound by
 // HBM with other workgroups to switch to): the registers stay at four
-// workgroups a CU or more.  MINW keeps the compiler to that.  384 tiles (1024 x 5504):
-// 29 -> 23 us; all of 133 M parameters: norm 186 -> 154 us, update 318 -> 279
-// (the small form there 309 and 356).
+// workgroups a CU or more.  MINW keeps the compiler to that.  us, one row at a
+// time -> this: 384 tiles (1024 x 5504) update 25 -> 19, 8192 tiles (16384 x
+// 8192) norm 115 -> 104, update 292 -> 241, 2048 tiles of 256 columns (half the
+// threads idle) update 28 -> 25, materialize 22 -> 20.
 template <int FU, int MINW>
 __global__ __launch_bounds__(256, MINW) void k_factored_apply(const uint8_t* __restrict__ meta, int action, float lr,
                                                         float decay, double* __restrict__ partials,
@@ -525,7 +526,6 @@ __global__ __launch_bounds__(256, MINW) void k_factored_apply(const uint8_t* __r
   const FTerm* terms = (const FTerm*)(params + hd->nparams);
   const int32_t* owners = (const int32_t*)(terms + hd->nterms);
   __shared__ float sl[FBM][FRMAX + 1];  // (left * scale) rows of this tile
-  __shared__ int ssel[FBM];             // the rows' places in a term's tail
   const long tile = blockIdx.x;
   const FParam P = params[owners[tile]];
   const long local = tile - P.first_tile;
@@ -588,31 +588,31 @@ __global__ __launch_bounds__(256, MINW) void k_factored_apply(const uint8_t* __r
     }
   }
   for (int ti = 0; ti < P.term_count; ti++) {
-    // the tile's tail places together (row by row each was a dependent load
-    // and a branch before the next one's), then the selected rows' loads
+    // the tile's tail places in one load (row by row each was a dependent load
+    // and a branch before the next one's), held as scalars by every wave, then
+    // the selected rows' loads; few rows are selected, so most tiles end here
     const FTerm tm = terms[P.term_begin + ti];
     const bool tvec = (tm.ld & 3) == 0 && al16(tm.right) && al16(tm.tail);
-    __syncthreads();
-    if (threadIdx.x < FBM) ssel[threadIdx.x] = m0 + threadIdx.x < P.rows ? tm.row_map[m0 + threadIdx.x] : -1;
-    __syncthreads();
+    const long mr = m0 + (threadIdx.x & (FBM - 1));
+    const int place = mr < P.rows ? tm.row_map[mr] : -1;
+    if (!__any(place >= 0)) continue;
+    int sel[FBM];
+#pragma unroll
+    for (int i = 0; i < FBM; i++) sel[i] = __builtin_amdgcn_readlane(place, i);
     if (cnt == 0) continue;
 #pragma unroll
     for (int i0 = 0; i0 < FBM; i0 += RU) {
       float4 tv[RU];
 #pragma unroll
-      for (int i = 0; i < RU; i++) {
-        const int sel = __builtin_amdgcn_readfirstlane(ssel[i0 + i]);
-        if (sel >= 0) tv[i] = ld4(tm.tail + (long)sel * tm.ld + n, cnt, tvec);
-      }
+      for (int i = 0; i < RU; i++)
+        if (sel[i0 + i] >= 0) tv[i] = ld4(tm.tail + (long)sel[i0 + i] * tm.ld + n, cnt, tvec);
 #pragma unroll
-      for (int i = 0; i < RU; i++) {
-        const int sel = __builtin_amdgcn_readfirstlane(ssel[i0 + i]);
-        if (sel >= 0) {
+      for (int i = 0; i < RU; i++)
+        if (sel[i0 + i] >= 0) {
           float4& q = g[i0 + i];
           q.x += tv[i].x * tm.scale; q.y += tv[i].y * tm.scale;
           q.z += tv[i].z * tm.scale; q.w += tv[i].w * tm.scale;
         }
-      }
     }
   }
   if (action == 2) {
